@@ -30,6 +30,9 @@ hipError_t launch_grid_build(const ScanArgs& a, int mol, const int* n, const dou
                              double4* out, hipStream_t st);
 hipError_t launch_scan_fast(const ScanArgs& a, bool f32, int comp, int G, int n_blocks, int W, int lds_sites,
                             bool scalar_sites, bool mid_family, hipStream_t st);
+size_t scan_iter_lds(int n_min, int n_max, int G, bool mid);
+hipError_t launch_scan_iter(const ScanArgs& a, int G, bool coul, bool grid, int n_blocks, int W, int n_min, int n_max,
+                            hipStream_t st);
 hipError_t launch_to_f32(const double4* in, float4* out, long n, hipStream_t st);
 hipError_t launch_record_totals(const DevRecord* rec, long n, int64_t* out, hipStream_t st);
 hipError_t noalloc_scratch_address(void** out);
@@ -416,11 +419,83 @@ static mafm_status build_tables(mafm_ctx* c, int n, const mafm_system_desc* sys,
 struct FastPlan {
     int G = 1, wps = 0, W = 1, n_blocks = 0, lds_sites = 0;
     bool scalar_sites = false, mid_family = false;
+    bool iter = false, coul = false, grid = false;   // the whole-iteration kernels (scan_iter.hip)
+    int n_min = 0;                                    // fewest sites of a molecule with columns
 };
 
 // LDS bytes the fast scan may stage one molecule's sites in
 static size_t scan_lds_limit(const mafm_ctx* c) {
     return c->lds_per_block > 1024 ? c->lds_per_block - 1024 : 0;
+}
+
+// Whether the whole-iteration kernels take these systems: FP64, one image,
+// Lennard-Jones (+ Coulomb) sites without an external potential or, for every
+// system, a force grid, and a Lennard-Jones dummy.
+static bool iter_systems(const mafm_ctx* c, const std::vector<long>& cols, bool& coul, bool& grid) {
+    bool sites = false;
+    coul = grid = false;
+    for (size_t m = 0; m < c->mols.size(); ++m) {
+        if (cols[m] <= 0) continue;
+        const DevMol& d = c->mols[m];
+        if (d.n_images > 1 || d.td_vdw != MAFM_VDW_LJ) return false;
+        if (d.force_grid >= 0) {
+            grid = true;
+            continue;
+        }
+        if (d.potential_grid >= 0 || d.n_seg[2] + d.n_seg[3] > 0) return false;
+        sites = true;
+        coul |= d.n_seg[0] > 0;
+    }
+    return sites != grid;
+}
+
+// Whether the whole-iteration kernels run this scan, and with how many lanes a
+// column (lanes = 0: chosen here).
+//
+// A wave's iteration costs about 45 instructions a site of a lane's share plus
+// 330 (groups of up to 8 lanes) or 250 for the rest, so few lanes a column do
+// the least work, and many columns at once want few lanes.  Against that: a
+// wave alone on its SIMD issues an FP64 instruction every 8 cycles, two waves
+// together one every 4 (measured), so up to one wave a SIMD the time is that of
+// one wave; two waves a SIMD take 1.35 times as long; and columns past the
+// 2 waves a SIMD that fit wait for a second round, the last of which is
+// partly empty.  The count with the least estimate is taken.  Measured, 96
+// charge-free sites, columns x lanes (ms): 2025 columns 64: 0.52, 32: 0.38,
+// 16: 0.43; 10 201 columns 32: 1.87, 16: 1.38, 8: 1.77; 16 384 columns 16:
+// 2.13, 8: 1.89, 4: 2.37 (two lanes of the general kernel: 2.99, 5.0, 5.0).
+static void plan_iter(const mafm_ctx* c, const std::vector<long>& cols, int lanes, bool mid, FastPlan& p) {
+    if (!iter_systems(c, cols, p.coul, p.grid)) return;
+    int n_max = 1;
+    long total = 0;
+    p.n_min = INT32_MAX;
+    for (size_t m = 0; m < c->mols.size(); ++m) {
+        if (cols[m] <= 0) continue;
+        total += cols[m];
+        n_max = std::max(n_max, (int)c->mols[m].n_sites);
+        p.n_min = std::min(p.n_min, (int)c->mols[m].n_sites);
+    }
+    if (!p.grid && (size_t)n_max * sizeof(SiteF64) > scan_lds_limit(c)) return;   // streamed, one lane a column
+    if (p.grid) {               // one corner of the cell a lane
+        p.iter = lanes == 0 || lanes == 8;
+        p.G = 8;
+        return;
+    }
+    const double simds = 4.0 * c->cus;
+    double best = 0;
+    for (int G = 4; G <= 64; G <<= 1) {
+        if (lanes > 0 && G != lanes) continue;
+        if (scan_iter_lds(p.n_min, n_max, G, mid) > scan_lds_limit(c)) continue;   // padding
+        double work = 0;        // instructions of an iteration, over the columns
+        for (size_t m = 0; m < c->mols.size(); ++m)
+            if (cols[m] > 0) work += (double)cols[m] * (45.0 * ((c->mols[m].n_sites + G - 1) / G) + (G <= 8 ? 330 : 250));
+        const double waves = std::ceil(total * (double)G / 64), rounds = waves / (2 * simds);
+        const double t = work / total * (waves <= simds ? 1.0 : 1.35 * std::max(1.0, 0.5 * (rounds + std::ceil(rounds))));
+        if (!p.iter || t < best) {
+            p.iter = true;
+            p.G = G;
+            best = t;
+        }
+    }
 }
 
 static mafm_status plan_fast(mafm_ctx* c, const mafm_scan_desc* d, bool f32, const std::vector<long>& cols, int lanes,
@@ -437,11 +512,15 @@ static mafm_status plan_fast(mafm_ctx* c, const mafm_scan_desc* d, bool f32, con
     for (const DevMol& m : c->mols) periodic |= m.n_images > 1;
     p.mid_family = d->minimiser == MAFM_MIN_FIRE && d->integrator == MAFM_INT_MIDPOINT && !periodic;
     p.wps = waves_per_simd > 0 ? waves_per_simd : (p.mid_family ? 3 : 2);
+    const bool mid = d->minimiser == MAFM_MIN_FIRE && d->integrator == MAFM_INT_MIDPOINT;
+    if (!f32) plan_iter(c, cols, lanes, mid, p);
     const long lanes_total = (long)c->cus * 4 * p.wps * 64;
     int64_t max_sites = 1;
     for (int m = 0; m < n_mols; ++m)
         if (cols[m] > 0) max_sites = std::max<int64_t>(max_sites, c->mols[m].force_grid >= 0 ? 1 : c->mols[m].n_sites);
-    if (lanes > 0) {
+    if (p.iter) {
+        // chosen above
+    } else if (lanes > 0) {
         p.G = lanes;
     } else {
         p.G = 1;
@@ -455,7 +534,7 @@ static mafm_status plan_fast(mafm_ctx* c, const mafm_scan_desc* d, bool f32, con
     // per pixel
     const size_t site_bytes = f32 ? sizeof(Site32) : sizeof(SiteF64);
     const size_t lds_limit = scan_lds_limit(c);
-    p.scalar_sites = (size_t)max_sites * site_bytes > lds_limit;
+    p.scalar_sites = !p.iter && (size_t)max_sites * site_bytes > lds_limit;
     if (p.scalar_sites && p.G > 1) {
         if (lanes > 0)
             return fail(c, MAFM_ERR_INVALID, "lanes_per_pixel > 1 needs the sites of one molecule to fit %zu bytes of LDS",
@@ -466,7 +545,14 @@ static mafm_status plan_fast(mafm_ctx* c, const mafm_scan_desc* d, bool f32, con
     // waves per workgroup share one LDS copy of the sites: grow W until the
     // LDS a CU holds admits wps waves per SIMD
     p.W = 1;
-    if (waves_per_group > 0) {
+    if (p.iter) {
+        // two waves a SIMD hold the resident sites; a force grid leaves room for three
+        if (waves_per_simd == 0) p.wps = p.grid ? 3 : 2;
+        const size_t bytes = p.grid ? 1 : scan_iter_lds(p.n_min, (int)max_sites, p.G, mid);
+        const long per_cu = (long)(c->lds_per_cu / bytes);
+        while (p.W < 8 && per_cu * p.W < 4L * p.wps) ++p.W;
+        if (waves_per_group > 0) p.W = waves_per_group;
+    } else if (waves_per_group > 0) {
         p.W = waves_per_group;
     } else if (!p.scalar_sites) {
         const size_t lds_bytes = std::max<size_t>((size_t)max_sites * site_bytes, 1);
@@ -1001,8 +1087,12 @@ static mafm_status scan_impl(mafm_ctx* c, const mafm_scan_desc* d, mafm_scan_sta
     } else {
         // 0 / 3: block-compensated (default), 1: Kahan, 2: plain FP32
         const int comp = d->compensation == 1 ? 1 : (d->compensation == 2 ? 0 : 2);
-        HIPCHK(c, launch_scan_fast(a, d->precision == MAFM_PREC_FAST32, comp, plan.G, plan.n_blocks, plan.W,
-                                   plan.lds_sites, plan.scalar_sites, plan.mid_family, c->stream));
+        if (plan.iter)
+            HIPCHK(c, launch_scan_iter(a, plan.G, plan.coul, plan.grid, plan.n_blocks, plan.W, plan.n_min,
+                                       plan.lds_sites, c->stream));
+        else
+            HIPCHK(c, launch_scan_fast(a, d->precision == MAFM_PREC_FAST32, comp, plan.G, plan.n_blocks, plan.W,
+                                       plan.lds_sites, plan.scalar_sites, plan.mid_family, c->stream));
     }
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     PendingScan ps;
