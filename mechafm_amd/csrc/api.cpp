@@ -30,8 +30,8 @@ hipError_t launch_grid_build(const ScanArgs& a, int mol, const int* n, const dou
                              double4* out, hipStream_t st);
 hipError_t launch_scan_fast(const ScanArgs& a, bool f32, int comp, int G, int n_blocks, int W, int lds_sites,
                             bool scalar_sites, bool mid_family, hipStream_t st);
-size_t scan_iter_lds(int n_min, int n_max, int G, bool mid);
-hipError_t launch_scan_iter(const ScanArgs& a, int G, bool coul, bool grid, int n_blocks, int W, int n_min, int n_max,
+size_t scan_iter_lds(int n_min, int n_max, int G, bool mid, bool images);
+hipError_t launch_scan_iter(const ScanArgs& a, int G, bool coul, int mode, int n_blocks, int W, int n_min, int n_max,
                             hipStream_t st);
 hipError_t launch_to_f32(const double4* in, float4* out, long n, hipStream_t st);
 hipError_t launch_record_totals(const DevRecord* rec, long n, int64_t* out, hipStream_t st);
@@ -419,7 +419,8 @@ static mafm_status build_tables(mafm_ctx* c, int n, const mafm_system_desc* sys,
 struct FastPlan {
     int G = 1, wps = 0, W = 1, n_blocks = 0, lds_sites = 0;
     bool scalar_sites = false, mid_family = false;
-    bool iter = false, coul = false, grid = false;   // the whole-iteration kernels (scan_iter.hip)
+    bool iter = false, coul = false;                  // the whole-iteration kernels (scan_iter.hip)
+    int mode = -1;                                    // iter_mode
     int n_min = 0;                                    // fewest sites of a molecule with columns
 };
 
@@ -428,43 +429,58 @@ static size_t scan_lds_limit(const mafm_ctx* c) {
     return c->lds_per_block > 1024 ? c->lds_per_block - 1024 : 0;
 }
 
-// Whether the whole-iteration kernels take these systems: FP64, one image,
-// Lennard-Jones (+ Coulomb) sites without an external potential or, for every
-// system, a force grid, and a Lennard-Jones dummy.
-static bool iter_systems(const mafm_ctx* c, const std::vector<long>& cols, bool& coul, bool& grid) {
-    bool sites = false;
-    coul = grid = false;
+// The nine image shifts are every sum of three along x and three along y (an
+// axis-aligned cell), x slowest.
+static bool product_images(const DevMol& d) {
+    if (d.n_images != 9) return false;
+    for (int k = 0; k < 9; ++k)
+        if (d.shift[k][0] != d.shift[3 * (k / 3)][0] || d.shift[k][1] != d.shift[k % 3][1] || d.shift[k][2] != 0) return false;
+    return true;
+}
+
+// Whether the whole-iteration kernels take these systems (FP64, Lennard-Jones
+// dummy), and in which mode: 0 Lennard-Jones (+ Coulomb) sites of one image
+// without an external potential, 1 force grids, 2 charge-free Lennard-Jones
+// sites with 3 x 3 product images, with or without a potential; -1 none.
+static int iter_mode(const mafm_ctx* c, const std::vector<long>& cols, bool& coul) {
+    int mode = -1;
+    coul = false;
     for (size_t m = 0; m < c->mols.size(); ++m) {
         if (cols[m] <= 0) continue;
         const DevMol& d = c->mols[m];
-        if (d.n_images > 1 || d.td_vdw != MAFM_VDW_LJ) return false;
-        if (d.force_grid >= 0) {
-            grid = true;
-            continue;
-        }
-        if (d.potential_grid >= 0 || d.n_seg[2] + d.n_seg[3] > 0) return false;
-        sites = true;
+        int mine;
+        if (d.td_vdw != MAFM_VDW_LJ) return -1;
+        if (d.force_grid >= 0) mine = 1;
+        else if (d.n_seg[2] + d.n_seg[3] > 0) return -1;
+        else if (d.n_images == 1 && d.potential_grid < 0) mine = 0;
+        else if (product_images(d) && d.n_seg[0] == 0) mine = 2;
+        else return -1;
+        if (mode >= 0 && mode != mine) return -1;
+        mode = mine;
         coul |= d.n_seg[0] > 0;
     }
-    return sites != grid;
+    return mode;
 }
 
 // Whether the whole-iteration kernels run this scan, and with how many lanes a
 // column (lanes = 0: chosen here).
 //
-// A wave's iteration costs about 45 instructions a site of a lane's share plus
+// A wave's iteration costs about 45 instructions a site of a lane's share (260
+// with its nine images) plus
 // 330 (groups of up to 8 lanes) or 250 for the rest, so few lanes a column do
 // the least work, and many columns at once want few lanes.  Against that: a
 // wave alone on its SIMD issues an FP64 instruction every 8 cycles, two waves
 // together one every 4 (measured), so up to one wave a SIMD the time is that of
 // one wave; two waves a SIMD take 1.35 times as long; and columns past the
 // 2 waves a SIMD that fit wait for a second round, the last of which is
-// partly empty.  The count with the least estimate is taken.  Measured, 96
+// partly empty; and the more columns share a wave, the longer its last ones
+// run alone (4 % a factor of two).  The count with the least estimate is taken.  Measured, 96
 // charge-free sites, columns x lanes (ms): 2025 columns 64: 0.52, 32: 0.38,
 // 16: 0.43; 10 201 columns 32: 1.87, 16: 1.38, 8: 1.77; 16 384 columns 16:
 // 2.13, 8: 1.89, 4: 2.37 (two lanes of the general kernel: 2.99, 5.0, 5.0).
 static void plan_iter(const mafm_ctx* c, const std::vector<long>& cols, int lanes, bool mid, FastPlan& p) {
-    if (!iter_systems(c, cols, p.coul, p.grid)) return;
+    p.mode = iter_mode(c, cols, p.coul);
+    if (p.mode < 0) return;
     int n_max = 1;
     long total = 0;
     p.n_min = INT32_MAX;
@@ -474,22 +490,25 @@ static void plan_iter(const mafm_ctx* c, const std::vector<long>& cols, int lane
         n_max = std::max(n_max, (int)c->mols[m].n_sites);
         p.n_min = std::min(p.n_min, (int)c->mols[m].n_sites);
     }
-    if (!p.grid && (size_t)n_max * sizeof(SiteF64) > scan_lds_limit(c)) return;   // streamed, one lane a column
-    if (p.grid) {               // one corner of the cell a lane
+    if (p.mode != 1 && (size_t)n_max * sizeof(SiteF64) > scan_lds_limit(c)) return;   // streamed, one lane a column
+    if (p.mode == 1) {               // one corner of the cell a lane
         p.iter = lanes == 0 || lanes == 8;
         p.G = 8;
         return;
     }
     const double simds = 4.0 * c->cus;
     double best = 0;
-    for (int G = 4; G <= 64; G <<= 1) {
+    const bool images = p.mode == 2;
+    const double site = images ? 260 : 45;
+    for (int G = images ? 8 : 4; G <= 64; G <<= 1) {
         if (lanes > 0 && G != lanes) continue;
-        if (scan_iter_lds(p.n_min, n_max, G, mid) > scan_lds_limit(c)) continue;   // padding
+        if (scan_iter_lds(p.n_min, n_max, G, mid, images) > scan_lds_limit(c)) continue;   // padding
         double work = 0;        // instructions of an iteration, over the columns
         for (size_t m = 0; m < c->mols.size(); ++m)
-            if (cols[m] > 0) work += (double)cols[m] * (45.0 * ((c->mols[m].n_sites + G - 1) / G) + (G <= 8 ? 330 : 250));
+            if (cols[m] > 0) work += (double)cols[m] * (site * ((c->mols[m].n_sites + G - 1) / G) + (G <= 8 ? 330 : 250));
         const double waves = std::ceil(total * (double)G / 64), rounds = waves / (2 * simds);
-        const double t = work / total * (waves <= simds ? 1.0 : 1.35 * std::max(1.0, 0.5 * (rounds + std::ceil(rounds))));
+        const double drain = 1 + 0.04 * std::log2(64.0 / G);
+        const double t = drain * work / total * (waves <= simds ? 1.0 : 1.35 * std::max(1.0, 0.5 * (rounds + std::ceil(rounds))));
         if (!p.iter || t < best) {
             p.iter = true;
             p.G = G;
@@ -547,10 +566,16 @@ static mafm_status plan_fast(mafm_ctx* c, const mafm_scan_desc* d, bool f32, con
     p.W = 1;
     if (p.iter) {
         // two waves a SIMD hold the resident sites; a force grid leaves room for three
-        if (waves_per_simd == 0) p.wps = p.grid ? 3 : 2;
-        const size_t bytes = p.grid ? 1 : scan_iter_lds(p.n_min, (int)max_sites, p.G, mid);
+        if (waves_per_simd == 0) p.wps = p.mode == 1 ? 3 : 2;
+        const size_t bytes = p.mode == 1 ? 1 : scan_iter_lds(p.n_min, (int)max_sites, p.G, mid, p.mode == 2);
         const long per_cu = (long)(c->lds_per_cu / bytes);
-        while (p.W < 8 && per_cu * p.W < 4L * p.wps) ++p.W;
+        // one wave a workgroup where the CU's LDS holds the copies of the waves it
+        // gets, else four (one a SIMD) or eight.  Images, 2000 sites: 900 columns
+        // in workgroups of 2 / 4 / 8 waves 21 / 13 / 20 ms, 4096 columns in two
+        // workgroups of 4 a CU 265, in one of 8 243 ms
+        const long waves = (total_cols * p.G + 63) / 64;
+        const long target = std::min(4L * p.wps, (waves + c->cus - 1) / c->cus);
+        if (per_cu < target) p.W = per_cu * 4 >= target && !(p.mode == 2 && target == 8) ? 4 : 8;
         if (waves_per_group > 0) p.W = waves_per_group;
     } else if (waves_per_group > 0) {
         p.W = waves_per_group;
@@ -1088,7 +1113,7 @@ static mafm_status scan_impl(mafm_ctx* c, const mafm_scan_desc* d, mafm_scan_sta
         // 0 / 3: block-compensated (default), 1: Kahan, 2: plain FP32
         const int comp = d->compensation == 1 ? 1 : (d->compensation == 2 ? 0 : 2);
         if (plan.iter)
-            HIPCHK(c, launch_scan_iter(a, plan.G, plan.coul, plan.grid, plan.n_blocks, plan.W, plan.n_min,
+            HIPCHK(c, launch_scan_iter(a, plan.G, plan.coul, plan.mode, plan.n_blocks, plan.W, plan.n_min,
                                        plan.lds_sites, c->stream));
         else
             HIPCHK(c, launch_scan_fast(a, d->precision == MAFM_PREC_FAST32, comp, plan.G, plan.n_blocks, plan.W,

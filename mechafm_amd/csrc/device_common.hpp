@@ -114,6 +114,7 @@ struct ScanArgs {
     // so the host may read the column's first k + 1 records as soon as it
     // sees the count.  Null: no counters.
     int32_t* col_done;
+    int32_t lds_sites;        // scan_iter.hip: sites the LDS copy has room for
 };
 
 // Heights [0, heights) of column `gcol` are in host memory (ScanArgs::col_done).

@@ -17,12 +17,14 @@
 // What bounds it now: FP64 issue (a lone wave issues an FP64 instruction every
 // 8 cycles, two waves one every 4) and, for few columns, the length of the
 // longest column's chain.
-// Measured (kernel ms, before -> now): one column over 96 sites 16.4 -> 3.2;
-// 101 x 101 columns x 41 heights over 96 charge-free sites 26.5 -> 12.4;
-// 33 x 33 columns, RK4, 131 charged sites 57 -> 16; 128 x 128 columns x 36
-// heights through a force grid 26.4 -> 7.1; 128 x 128 x 30 over 150 charged
-// sites 54.9 -> 23; 64 molecules of 20 to 400 sites, 64 x 64 x 40 each 406 ->
-// 386.
+// Measured (kernel ms, before -> now):
+//   one column over 96 sites                                      16.4 -> 3.2
+//   101 x 101 columns x 41 heights, 96 charge-free sites          26.5 -> 12.4
+//   33 x 33 x 41, RK4, 131 charged sites                          57 -> 16
+//   128 x 128 x 36 through a force grid                           26.4 -> 7.1
+//   128 x 128 x 30, 150 charged sites                             54.9 -> 23
+//   64 molecules of 20 to 400 charged sites, 64 x 64 x 40 each    406 -> 386
+//   64 x 64 x 40, 2000 sites with nine images and a potential     437 -> 244
 #include "../../include/mafm.h"
 #include <type_traits>
 
@@ -147,6 +149,66 @@ __device__ inline void pair_acc(const SiteLJ& st, double tx, double ty, double t
     acc[2] = fma(fs, dz, acc[2]);
 }
 
+// One charge-free site and its 3 x 3 images: ax[i] / ay[j] = tip minus the
+// images' shift along x / y.  The squared distances are sums of three and
+// three parts, the nine reciprocals come from one hardware reciprocal (the
+// product of all, refined, times the products of the others: 30 instructions
+// instead of 54), and the force's components are sums of row and column sums:
+// 13.3 instructions a pair instead of 20.
+template <bool E>
+__device__ inline void images_acc(const double4& st, double q1, const double* ax, const double* ay, double pz, double* acc) {
+    const double dz = pz - st.z, dz2 = dz * dz;
+    double dx[3], dy[3], xz[3], yy[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        dx[i] = ax[i] - st.x;
+        xz[i] = fma(dx[i], dx[i], dz2);
+        dy[i] = ay[i] - st.y;
+        yy[i] = dy[i] * dy[i];
+    }
+    double r2[3][3], p01[3], row[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) r2[i][j] = xz[i] + yy[j];
+        p01[i] = r2[i][0] * r2[i][1];
+        row[i] = p01[i] * r2[i][2];
+    }
+    const double q01 = row[0] * row[1];
+    const double all = rcp64h(q01 * row[2]);
+    const double t2 = all * row[2];
+    const double irow[3] = {t2 * row[1], t2 * row[0], all * q01};
+    double cy[3], sum = 0, s6 = 0, sg = 0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const double t = irow[i] * r2[i][2];
+        const double ir2[3] = {t * r2[i][1], t * r2[i][0], irow[i] * p01[i]};
+        double rx = 0;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const double ir6 = ir2[j] * ir2[j] * ir2[j];
+            const double gl = fma(q1, ir6, -st.w) * ir6;
+            const double fs = gl * ir2[j];
+            rx = j ? rx + fs : fs;
+            cy[j] = i ? cy[j] + fs : fs;
+            if (E) {
+                s6 += ir6;
+                sg += gl;
+            }
+        }
+        acc[0] = fma(dx[i], rx, acc[0]);
+        sum += rx;
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) acc[1] = fma(dy[j], cy[j], acc[1]);
+    acc[2] = fma(dz, sum, acc[2]);
+    if (E) acc[3] = fma(-st.w, s6, acc[3] + sg);   // 12 E = sum of ir6 (fl - 6 es6)
+}
+// x, or 1e15 with its sign where it is finite and larger
+__device__ inline double keep_near(double x) {
+    return fabs(x) > 1e15 && fabs(x) < INFINITY ? copysign(1e15, x) : x;
+}
+
 // Tip-dummy constants of the workgroup's molecule
 struct Dummy {
     double p0, p1, qq, k, r0, kk;
@@ -213,10 +275,17 @@ struct Grid {
     cptr<DevGrid> d;
 };
 
+// What a column's tip-surface force is made of: the molecule's sites, a force
+// grid, or the sites' 3 x 3 periodic images and, where the system has one, an
+// external potential.
+enum { ITER_SITES = 0, ITER_GRID = 1, ITER_IMAGES = 2 };
+
 // Sites of a lane that shares n sites with G - 1 others, padded: at least the
-// resident ones, and a multiple of two past them.
+// resident ones, and a multiple of two past them (res = 1, the images' kernels:
+// no padding of the share).
 __host__ __device__ inline int padded_share(int n, int G, int res) {
     const int per = (n + G - 1) / G;
+    if (res == 1) return per > 1 ? per : 1;
     return res + (per > res ? (per - res + 1) / 2 * 2 : 0);
 }
 // The resident count for molecules of n sites or more: a lane's whole share up
@@ -230,8 +299,9 @@ inline int resident_sites(int n, int G, bool mid) {
 // RES of a lane's sites stay in registers for the whole scan (the first RES
 // of its share, loaded from the staged copy); the others stream from LDS two
 // at a time.
-template <int G, int RES, bool COUL, bool GRID, bool MID>
+template <int G, int RES, bool COUL, int MODE, bool MID>
 __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanArgs& a) {
+    constexpr bool GRID = MODE == ITER_GRID, IMG = MODE == ITER_IMAGES;
     const int lane = threadIdx.x & 63;
     const int gl = Lanes<G>::place(lane);
     const bool leader = gl == 0;
@@ -240,16 +310,21 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
     extern __shared__ double2 lds_iter[];
     __shared__ int next_shared;
     SiteLJ* const lsite = reinterpret_cast<SiteLJ*>(lds_iter);
+    // the images' kernels: {x, y, z, q0} and, behind the most sites of a molecule, q1 (40 B a site)
+    double4* const lxyz = reinterpret_cast<double4*>(lds_iter);
+    double* const lq1 = reinterpret_cast<double*>(lds_iter) + 4 * (size_t)a.lds_sites;
 
     int rk = __builtin_amdgcn_readfirstlane(pick_rank(a, blockIdx.x, gridDim.x));
     int m = a.mol_order[rk];
-    SiteLJ res[RES];
+    SiteLJ res[RES > 0 ? RES : 1];
     Dummy D;
     int per_lane = 0;                 // sites of a lane, a multiple of two past the resident ones
     // the corners last read, for the half steps and the full steps apart: a
     // pair of points on both sides of a cell face does not reload each other's
     Corner cn0 = {{0, 0, 0, 0}, -1}, cn1 = cn0;
     Grid g;
+    bool has_grid = false;
+    double img_x[3], img_y[3];        // the images' shifts along x and y
     const int bit[3] = {gl >> 2 & 1, gl >> 1 & 1, gl & 1};
     const double wsign[3] = {bit[0] ? 1.0 : -1.0, bit[1] ? 1.0 : -1.0, bit[2] ? 1.0 : -1.0};
     const double wbase[3] = {1.0 - bit[0], 1.0 - bit[1], 1.0 - bit[2]};
@@ -258,8 +333,9 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
         D.p0 = M->td_p0; D.p1 = M->td_p1; D.qq = M->td_qq; D.k = M->td_k; D.r0 = M->td_r0;
         D.kk = 2 * D.k;
         D.coul = M->td_coul != 0;
-        if (GRID) {
-            g.d = as_const(a.grids) + M->force_grid;
+        has_grid = GRID || (IMG && M->potential_grid >= 0);
+        if (has_grid) {
+            g.d = as_const(a.grids) + (GRID ? M->force_grid : M->potential_grid);
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
                 g.off[d] = g.d->offset[d];
@@ -272,7 +348,14 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
             g.near = (long)g.n[0] * g.n[1] < (1 << 24) && g.n[2] < (1 << 24) &&
                      (long)g.n[0] * g.n[1] * g.n[2] < INT32_MAX;
             cn0.idx = cn1.idx = -1;
-            return;
+        }
+        if (GRID) return;
+        if (IMG) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                img_x[d] = M->shift[3 * d][0];
+                img_y[d] = M->shift[d][1];
+            }
         }
         const int n = M->n_seg[0] + M->n_seg[1];
         per_lane = padded_share(n, G, RES);
@@ -281,16 +364,22 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
             SiteLJ s = {1e4, 1e4, 1e4, 0, 0, 0};     // padding: no force, finite distance
             if (t < n) {
                 const SiteF64 f = a.segf64[M->seg_off + t];
-                s.x = f.x + M->shift[0][0]; s.y = f.y + M->shift[0][1]; s.z = f.z + M->shift[0][2];
+                s.x = f.x; s.y = f.y; s.z = f.z;
+                if (!IMG) { s.x += M->shift[0][0]; s.y += M->shift[0][1]; s.z += M->shift[0][2]; }
                 s.q0 = COUL ? f.p0 * 0x1p-8 : f.p0;
                 s.q1 = COUL ? f.p1 * 0x1p-14 : f.p1;
                 s.qc = f.qq * -0x1p-3;
             }
-            lsite[t] = s;
+            if (IMG) {
+                lxyz[t] = make_double4(s.x, s.y, s.z, s.q0);
+                lq1[t] = s.q1;
+            } else {
+                lsite[t] = s;
+            }
         }
         __syncthreads();
 #pragma unroll
-        for (int u = 0; u < RES; ++u) res[u] = lsite[u * G + gl];
+        for (int u = 0; u < (IMG ? 0 : RES); ++u) res[u] = lsite[u * G + gl];
     };
     stage(m);
 
@@ -308,57 +397,96 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
     int64_t trips = 0;
     int32_t active = 0;
 
-    // tip-surface force and energy at p, summed over the group's lanes
-    auto surface = [&](auto want_e, Corner& cn, double px, double py, double pz, double* r) {
-        constexpr bool E = decltype(want_e)::value;
-        r[3] = 0;
-        if (GRID) {
-            double q[3];
-            if (g.diagonal) {
-                q[0] = (px - g.off[0]) * g.inv[0];
-                q[1] = (py - g.off[1]) * g.inv[1];
-                q[2] = (pz - g.off[2]) * g.inv[2];
-            } else {
-                mat_vec(g.d->inv, px - g.off[0], py - g.off[1], pz - g.off[2], q[0], q[1], q[2]);
-            }
-            int gp[3], at[3], fl = 0;
-            bool inside = true;
+    // this lane's corner of the grid cell around p: its weight, the samples in
+    // cn.v; counts: the point is one of the column's evaluations, so leaving
+    // the grid is noted
+    auto corner = [&](Corner& cn, bool counts, double px, double py, double pz) {
+        double q[3];
+        if (g.diagonal) {
+            q[0] = (px - g.off[0]) * g.inv[0];
+            q[1] = (py - g.off[1]) * g.inv[1];
+            q[2] = (pz - g.off[2]) * g.inv[2];
+        } else {
+            mat_vec(g.d->inv, px - g.off[0], py - g.off[1], pz - g.off[2], q[0], q[1], q[2]);
+        }
+        int gp[3], at[3], fl = 0;
+        bool inside = true;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            gp[d] = (int)floor(q[d]);
+            at[d] = gp[d] + bit[d];
+            inside &= (unsigned)gp[d] < (unsigned)(g.n[d] - 1);
+        }
+        if (!inside) {   // the clamp and wrap rules of grid_lookup
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
-                gp[d] = (int)floor(q[d]);
-                at[d] = gp[d] + bit[d];
-                inside &= (unsigned)gp[d] < (unsigned)(g.n[d] - 1);
-            }
-            if (!inside) {   // the clamp and wrap rules of grid_lookup
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    const int n = g.n[d];
-                    if (!g.periodic) {
-                        if (gp[d] < 0) { gp[d] = 0; fl |= REC_GRID_CLAMP; }
-                        else if (gp[d] >= n) { gp[d] = n - 1; fl |= REC_GRID_CLAMP; }
-                        if (gp[d] + 1 >= n) fl |= REC_OUT_OF_GRID;
-                    }
-                    int i = gp[d] + bit[d];
-                    if (g.periodic && (i < 0 || i >= n)) i -= (int)floor((double)i / n) * n;
-                    at[d] = i < 0 ? 0 : (i >= n ? n - 1 : i);   // inside the grid even for non-finite positions
+                const int n = g.n[d];
+                if (!g.periodic) {
+                    if (gp[d] < 0) { gp[d] = 0; fl |= REC_GRID_CLAMP; }
+                    else if (gp[d] >= n) { gp[d] = n - 1; fl |= REC_GRID_CLAMP; }
+                    if (gp[d] + 1 >= n) fl |= REC_OUT_OF_GRID;
                 }
-                flags |= fl;
+                int i = gp[d] + bit[d];
+                if (g.periodic && (i < 0 || i >= n)) i -= (int)floor((double)i / n) * n;
+                at[d] = i < 0 ? 0 : (i >= n ? n - 1 : i);   // inside the grid even for non-finite positions
             }
-            // f on an upper corner, 1 - f on a lower one, each rounded once
-            const double w = fma(q[0] - gp[0], wsign[0], wbase[0]) * fma(q[1] - gp[1], wsign[1], wbase[1]) *
-                             fma(q[2] - gp[2], wsign[2], wbase[2]);
-            long idx;
-            if (g.near) idx = (int)(__umul24(__umul24(at[0], g.n[1]) + at[1], g.n[2]) + at[2]);
-            else idx = ((long)at[0] * g.n[1] + at[1]) * g.n[2] + at[2];
-            if (idx != cn.idx) {
-                cn.v = g.fe[idx];
-                cn.idx = idx;
-            }
+            if (counts) flags |= fl;
+        }
+        // f on an upper corner, 1 - f on a lower one, each rounded once
+        const double w = fma(q[0] - gp[0], wsign[0], wbase[0]) * fma(q[1] - gp[1], wsign[1], wbase[1]) *
+                         fma(q[2] - gp[2], wsign[2], wbase[2]);
+        long idx;
+        if (g.near) idx = (int)(__umul24(__umul24(at[0], g.n[1]) + at[1], g.n[2]) + at[2]);
+        else idx = ((long)at[0] * g.n[1] + at[1]) * g.n[2] + at[2];
+        if (idx != cn.idx) {
+            cn.v = g.fe[idx];
+            cn.idx = idx;
+        }
+        return w;
+    };
+    // tip-surface force and energy at p, summed over the group's lanes
+    auto surface = [&](auto want_e, Corner& cn, bool counts, double px, double py, double pz, double* r) {
+        constexpr bool E = decltype(want_e)::value;
+        r[3] = 0;
+        if constexpr (GRID) {
+            const double w = corner(cn, counts, px, py, pz);
             r[0] = w * cn.v.x;
             r[1] = w * cn.v.y;
             r[2] = w * cn.v.z;
             if (E) r[3] = w * cn.v.w;
             group_sums<G, E ? 4 : 3>(r);
+        } else if constexpr (IMG) {
+            r[0] = r[1] = r[2] = 0;
+            if (has_grid && gl < 8) {   // eight of the column's lanes hold the potential's corners
+                const double w = corner(cn, counts, px, py, pz);
+                r[0] = w * cn.v.x;
+                r[1] = w * cn.v.y;
+                r[2] = w * cn.v.z;
+                if (E) r[3] = 12.0 * w * cn.v.w;
+            }
+            // a tip thrown past 1e15 A feels nothing here; nearer, it keeps the
+            // product of nine squared distances inside the exponent range
+            if (__any(fmax(fmax(fabs(px), fabs(py)), fabs(pz)) > 1e15)) {
+                px = keep_near(px);
+                py = keep_near(py);
+                pz = keep_near(pz);
+            }
+            const double ax[3] = {px - img_x[0], px - img_x[1], px - img_x[2]};
+            const double ay[3] = {py - img_y[0], py - img_y[1], py - img_y[2]};
+            int t = gl;
+            double4 st = lxyz[t];
+            double q1 = lq1[t];
+            for (int u = 1; u < per_lane; ++u) {
+                t += G;
+                const double4 st2 = lxyz[t];
+                const double q2 = lq1[t];
+                images_acc<E>(st, q1, ax, ay, pz, r);
+                st = st2;
+                q1 = q2;
+            }
+            images_acc<E>(st, q1, ax, ay, pz, r);
+            group_sums<G, E ? 4 : 3>(r);
+            if (E) r[3] *= 1.0 / 12.0;
         } else {
             r[0] = r[1] = r[2] = 0;
 #pragma unroll
@@ -391,11 +519,11 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
         }
     };
     // the whole list: tip-surface plus, where with_d, tip-dummy
-    auto total = [&](auto want_e, Corner& cn, bool with_d, double px, double py, double pz, double* r) {
+    auto total = [&](auto want_e, Corner& cn, bool counts, bool with_d, double px, double py, double pz, double* r) {
         constexpr bool E = decltype(want_e)::value;
         double d[4];
         dummy_terms<E>(D, dmx, dmy, dmz, px, py, pz, d);
-        surface(want_e, cn, px, py, pz, r);
+        surface(want_e, cn, counts, px, py, pz, r);
 #pragma unroll
         for (int q = 0; q < (E ? 4 : 3); ++q) r[q] += with_d ? d[q] : 0.0;
     };
@@ -522,13 +650,13 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
             // finished height at theirs (tip-surface terms only)
             const double hx = dt / 2 * vx, hy = dt / 2 * vy, hz = dt / 2 * vz;
             if (__any(emits)) {
-                total(std::true_type{}, cn0, !emits, tx, ty, tz, r);
+                total(std::true_type{}, cn0, true, !emits, tx, ty, tz, r);
                 if (emits) emit(r);
             } else {
-                total(std::false_type{}, cn0, true, tx, ty, tz, r);
+                total(std::false_type{}, cn0, true, true, tx, ty, tz, r);
             }
             const double ax = fma(dt / 2, r[0], vx), ay = fma(dt / 2, r[1], vy), az = fma(dt / 2, r[2], vz);
-            total(std::true_type{}, cn1, true, tx + hx, ty + hy, tz + hz, r);
+            total(std::true_type{}, cn1, live, true, tx + hx, ty + hy, tz + hz, r);
             if (live) {
                 tx = fma(dt, ax, tx); ty = fma(dt, ay, ty); tz = fma(dt, az, tz);
                 vx = fma(dt, r[0], vx); vy = fma(dt, r[1], vy); vz = fma(dt, r[2], vz);
@@ -543,7 +671,7 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
             double bx = 0, by = 0, bz = 0, cx = 0, cy = 0, cz = 0, ce = 0;    // sums over the stages
             const int ns = rk4 ? 4 : 1;
             for (int s = 0; s < ns; ++s) {
-                total(std::true_type{}, cn0, s > 0 || !emits, px, py, pz, r);
+                total(std::true_type{}, cn0, s == 0 || live, s > 0 || !emits, px, py, pz, r);
                 if (s == 0 && __any(emits)) {
                     if (emits) emit(r);
                     if (!__any(live)) break;
@@ -588,10 +716,12 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
     if (leader && active) atomicAdd((unsigned long long*)&a.counters[5], (unsigned long long)active);
 }
 
-template <int G, int RES, bool COUL, bool GRID, bool MID>
+template <int G, int RES, bool COUL, int MODE, bool MID>
 __global__ void __launch_bounds__(512, 2) k_scan_iter(ScanArgs a) {
-    scan_iter_body<G, RES, COUL, GRID, MID>(a);
+    scan_iter_body<G, RES, COUL, MODE, MID>(a);
 }
+
+size_t site_bytes(int mode) { return mode == ITER_IMAGES ? 40 : sizeof(SiteLJ); }
 
 struct IterLaunch {
     const ScanArgs& a;
@@ -600,22 +730,24 @@ struct IterLaunch {
     hipStream_t st;
 };
 
-template <int G, int RES, bool COUL, bool GRID, bool MID>
+template <int G, int RES, bool COUL, int MODE, bool MID>
 hipError_t launch_one(const IterLaunch& L) {
-    const size_t lds = GRID ? 0 : sizeof(SiteLJ) * (size_t)G * padded_share(L.n_max, G, RES);
-    const auto fn = &k_scan_iter<G, RES, COUL, GRID, MID>;
+    const size_t lds = MODE == ITER_GRID ? 0 : site_bytes(MODE) * (size_t)G * padded_share(L.n_max, G, RES);
+    const auto fn = &k_scan_iter<G, RES, COUL, MODE, MID>;
     if (lds > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(fn, dim3(L.n_blocks), dim3(64 * L.W), lds, L.st, L.a);
+    ScanArgs a = L.a;
+    a.lds_sites = G * padded_share(L.n_max, G, RES);
+    hipLaunchKernelGGL(fn, dim3(L.n_blocks), dim3(64 * L.W), lds, L.st, a);
     return hipGetLastError();
 }
 
-template <int G, int RES, bool COUL, bool GRID = false>
+template <int G, int RES, bool COUL, int MODE = ITER_SITES>
 hipError_t launch_mid(const IterLaunch& L) {
-    return L.mid ? launch_one<G, RES, COUL, GRID, true>(L) : launch_one<G, RES, COUL, GRID, false>(L);
+    return L.mid ? launch_one<G, RES, COUL, MODE, true>(L) : launch_one<G, RES, COUL, MODE, false>(L);
 }
 
 template <int G, bool COUL>
@@ -627,7 +759,7 @@ hipError_t launch_res(const IterLaunch& L) {
         case 5: return launch_mid<G, 5, COUL>(L);
         case 6: return launch_mid<G, 6, COUL>(L);
         default:
-            if constexpr (G <= 8) return launch_one<G, 8, COUL, false, true>(L);
+            if constexpr (G <= 8) return launch_one<G, 8, COUL, ITER_SITES, true>(L);
             return hipErrorInvalidValue;
     }
 }
@@ -647,19 +779,28 @@ hipError_t launch_g(const IterLaunch& L, int G) {
 }  // namespace
 
 // LDS bytes of one workgroup that scans molecules of n_min to n_max sites
-size_t scan_iter_lds(int n_min, int n_max, int G, bool mid) {
-    return sizeof(SiteLJ) * (size_t)G * padded_share(n_max, G, resident_sites(n_min, G, mid));
+size_t scan_iter_lds(int n_min, int n_max, int G, bool mid, bool images) {
+    return site_bytes(images ? ITER_IMAGES : ITER_SITES) * (size_t)G * padded_share(n_max, G, images ? 1 : resident_sites(n_min, G, mid));
 }
 
 // n_blocks workgroups of W waves (W = 1 .. 8), G lanes a pixel column (4 ..
-// 64); coul: some site carries a charge; grid: every molecule is a force grid
-// (G = 8, the sites unused)
-hipError_t launch_scan_iter(const ScanArgs& a, int G, bool coul, bool grid, int n_blocks, int W, int n_min, int n_max,
+// 64; a force grid 8, periodic images 8 .. 64); coul: some site carries a
+// charge; mode: ITER_*
+hipError_t launch_scan_iter(const ScanArgs& a, int G, bool coul, int mode, int n_blocks, int W, int n_min, int n_max,
                             hipStream_t st) {
     if (W < 1 || W > 8) return hipErrorInvalidValue;
     const IterLaunch L = {a, a.minimiser != MAFM_MIN_SD && a.integrator == MAFM_INT_MIDPOINT, n_blocks, W, n_min, n_max,
                           st};
-    if (grid) return G == 8 ? launch_mid<8, 2, false, true>(L) : hipErrorInvalidValue;
+    if (mode == ITER_GRID) return G == 8 ? launch_mid<8, 2, false, ITER_GRID>(L) : hipErrorInvalidValue;
+    if (mode == ITER_IMAGES) {
+        switch (G) {
+            case 8: return launch_mid<8, 1, false, ITER_IMAGES>(L);
+            case 16: return launch_mid<16, 1, false, ITER_IMAGES>(L);
+            case 32: return launch_mid<32, 1, false, ITER_IMAGES>(L);
+            case 64: return launch_mid<64, 1, false, ITER_IMAGES>(L);
+            default: return hipErrorInvalidValue;
+        }
+    }
     return coul ? launch_g<true>(L, G) : launch_g<false>(L, G);
 }
 

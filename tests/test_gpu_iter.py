@@ -125,3 +125,39 @@ def test_force_grid(gpu_ctx, periodic, skew):
     empty, keep2 = _system(0, False, np.random.default_rng(1))
     gpu_ctx.set_systems([empty])
     gpu_ctx.grid_free(h)
+
+
+@pytest.mark.parametrize("potential", [False, True])
+@pytest.mark.parametrize("n", [1, 9, 64, 130])
+def test_periodic_images(gpu_ctx, n, potential):
+    """3 x 3 images of an axis-aligned cell (nine reciprocals from one), with
+    and without an external potential, and the general kernel for shifts that
+    are no product; a periodic system's bars are those of the others."""
+    rng = np.random.default_rng(n)
+    cell = np.array([7.0, 6.0, 20.0])
+    d, keep = _system(n, False, rng)
+    h = -1
+    if potential:
+        g = (8, 6, 40)
+        h = gpu_ctx.grid_upload(g, np.diag(cell / g), np.zeros(3), rng.normal(0, 0.05, (int(np.prod(g)), 4)), True)
+    d.potential_grid, d.tip_pbc = h, 1
+    for k in range(3):
+        d.cell[4 * k] = cell[k]
+    shifts = np.array([[i * cell[0], j * cell[1], 0.0] for i in (-1, 0, 1) for j in (-1, 0, 1)])
+    for sh, product in ((shifts, True), (shifts + np.array([[0.0, 0.5 * (k // 3), 0.0] for k in range(9)]), False)):
+        d.n_images, d.image_shifts = 9, sh.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+        gpu_ctx.set_systems([d])
+        gpu_ctx.scan(_desc(4, 3, 5, "plain64"))
+        want = gpu_ctx.records(0, 60)
+        for lanes in (0, 8, 16, 32, 64):
+            gpu_ctx.scan(_desc(4, 3, 5, "fast64", lanes))
+            got = gpu_ctx.records(0, 60)
+            np.testing.assert_array_equal(got["n_steps"], want["n_steps"])
+            np.testing.assert_array_equal(got["flags"], want["flags"])
+            big = max(np.abs(want[f]).max() for f in ("fx", "fy", "fz"))
+            for f in ("rx", "ry", "rz", "fx", "fy", "fz", "e"):
+                assert np.abs(got[f] - want[f]).max() <= 1e-8 * max(big, 1.0)
+    if potential:
+        empty, keep2 = _system(0, False, rng)
+        gpu_ctx.set_systems([empty])
+        gpu_ctx.grid_free(h)
