@@ -194,7 +194,7 @@ struct mafm_ctx {
     bool host_pending = false;     // launched, not yet ended by mafm_scan_host_wait
     PendingScan pending;
     // flexible scan: term list, index tables, initial positions, kept states, per-block work
-    DevBuf<mafm_flex_term> d_fx_terms;
+    DevBuf<FxTerm> d_fx_terms;
     DevBuf<int32_t> d_fx_ints;
     DevBuf<double> d_fx_pos, d_fx_state, d_fx_work;
     DevBuf<double> d_sys;          // System operators: positions, velocities, forces, energies, steps
@@ -1216,28 +1216,29 @@ static bool flex_tip_surface(const mafm_flex_term& t) {   // isTipSurface (inter
     return (t.kind == MAFM_FX_LJ || t.kind == MAFM_FX_MORSE || t.kind == MAFM_FX_COULOMB) && t.atom[0] == 1;
 }
 
-// Relative length of one term evaluation's dependent chain by kind (square
-// roots, IEEE divisions and libm calls set it: a dihedral has three roots,
-// seven divisions and an atan, an angle an acos, a Morse term an exp).
+// Relative cost of one term evaluation by kind, from its instructions (a
+// dihedral has three roots, seven divisions and an atan, an angle two roots, 16
+// divisions, an acos and a sin, a Morse term an exp).
 static double flex_cost(int kind) {
     switch (kind) {
-        case MAFM_FX_DIHEDRAL: return 16;
-        case MAFM_FX_ANGLE: return 8;
-        case MAFM_FX_MORSE: return 5;
-        case MAFM_FX_SUBSTRATE: return 4;
-        case MAFM_FX_XY_HARMONIC: return 1;
-        default: return 3;
+        case MAFM_FX_DIHEDRAL: return 33;
+        case MAFM_FX_ANGLE: return 40;
+        case MAFM_FX_MORSE: return 10;
+        case MAFM_FX_SUBSTRATE: case MAFM_FX_BOND: return 6;
+        case MAFM_FX_XY_HARMONIC: return 3;
+        default: return 5;
     }
 }
 
-// Which terms each thread of a `waves`-wavefront block evaluates (the
-// FlexArgs::sched table): the terms of each kind, in list order, are cut
-// into wave-rounds of 64, so the 64 lanes of a round run one code path, and
-// the rounds are dealt longest first, each to the wave with the least work
-// so far.  Returns the number of rounds.
-static int flex_schedule(const std::vector<mafm_flex_term>& eval, int waves, std::vector<int32_t>& sched) {
+// The records of `terms` in the order the threads of a `waves`-wavefront block
+// evaluate them (FlexArgs::terms): the terms of each kind, in list order, are
+// cut into wave-rounds of 64, so the 64 lanes of a round run one code path, and
+// the rounds are dealt longest first, each to the wave with the least work so
+// far.  The last wave starts with `head` (it sums FIRE's power first).  Returns
+// the number of rounds.
+static int flex_schedule(const std::vector<FxTerm>& terms, int waves, double head, std::vector<FxTerm>& out) {
     std::map<int, std::vector<int32_t>> by_kind;
-    for (int k = 0; k < (int)eval.size(); ++k) by_kind[eval[k].kind].push_back(k);
+    for (int k = 0; k < (int)terms.size(); ++k) by_kind[terms[k].kind].push_back(k);
     struct Round {
         double cost;
         const int32_t* terms;
@@ -1249,6 +1250,7 @@ static int flex_schedule(const std::vector<mafm_flex_term>& eval, int waves, std
             rounds.push_back({flex_cost(kv.first), kv.second.data() + q, (int)std::min<size_t>(64, kv.second.size() - q)});
     std::stable_sort(rounds.begin(), rounds.end(), [](const Round& x, const Round& y) { return x.cost > y.cost; });
     std::vector<double> load(waves, 0.0);
+    load[waves - 1] = head;
     std::vector<std::vector<int>> mine(waves);
     for (int r = 0; r < (int)rounds.size(); ++r) {
         const int w = (int)(std::min_element(load.begin(), load.end()) - load.begin());
@@ -1258,13 +1260,91 @@ static int flex_schedule(const std::vector<mafm_flex_term>& eval, int waves, std
     int n_rounds = 0;
     for (const auto& m : mine) n_rounds = std::max(n_rounds, (int)m.size());
     const int T = 64 * waves;
-    sched.assign((size_t)n_rounds * T, -1);
+    FxTerm none;
+    memset(&none, 0, sizeof none);
+    none.kind = -1;
+    out.assign((size_t)n_rounds * T, none);
     for (int w = 0; w < waves; ++w)
         for (int r = 0; r < (int)mine[w].size(); ++r) {
             const Round& R = rounds[mine[w][r]];
-            for (int l = 0; l < R.n; ++l) sched[(size_t)r * T + 64 * w + l] = R.terms[l];
+            for (int l = 0; l < R.n; ++l) out[(size_t)r * T + 64 * w + l] = terms[R.terms[l]];
         }
     return n_rounds;
+}
+
+// Device records of an interaction list: every term that acts on an atom whose
+// force is summed, its result slots (numbered per atom in the order
+// Interaction::eval adds to forces_[i]) and its places in the tip's energy list
+// (in the order it adds to energies_[1]).  idx: the kernels' index tables.
+struct FlexList {
+    std::vector<FxTerm> terms;
+    std::vector<int32_t> idx;
+    int n_slots = 0, n_tip = 0, tip_rank = 0;
+    int tip_ts_slots = 0, tip_ts_terms = 0;   // of the first n_ts terms
+};
+
+static FlexList flex_list(int n, int n_terms, const mafm_flex_term* terms, int n_ts, const int32_t* fixed,
+                          const std::vector<char>& summed) {
+    FlexList L;
+    std::vector<int32_t> cnt(n, 0), order(n), rank(n);
+    for (int k = 0; k < n_terms; ++k)
+        for (int r = 0; r < flex_arity(terms[k].kind); ++r) cnt[terms[k].atom[r]] += summed[terms[k].atom[r]];
+    for (int i = 0; i < n; ++i) {
+        order[i] = i;
+        L.n_slots += cnt[i];
+    }
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cnt[x] > cnt[y]; });
+    for (int k = 0; k < n; ++k) rank[order[k]] = k;
+    L.tip_rank = rank[1];
+    // row q: the q-th slots of the atoms that have more than q
+    std::vector<int32_t> row(cnt[order[0]] + 8, 0);
+    int width = n, at = 0;
+    for (int q = 0; q < cnt[order[0]]; ++q) {
+        while (width > 0 && cnt[order[width - 1]] <= q) --width;
+        row[q] = at;
+        at += 3 * width;
+    }
+    for (int k = 0; k < n; ++k) L.idx.push_back(cnt[order[k]]);
+    L.idx.insert(L.idx.end(), order.begin(), order.end());
+    L.idx.insert(L.idx.end(), fixed, fixed + n);
+    L.idx.insert(L.idx.end(), row.begin(), row.end());
+    std::vector<int32_t> next(n, 0);
+    for (int k = 0; k < n_terms; ++k) {
+        const mafm_flex_term& T = terms[k];
+        const int ar = flex_arity(T.kind);
+        FxTerm f;
+        memset(&f, 0, sizeof f);
+        f.kind = T.kind;
+        for (int r = 0; r < 4; ++r) {
+            f.atom[r] = r < ar ? T.atom[r] : 0;
+            f.slot[r] = 3 * L.n_slots;
+        }
+        f.place[0] = f.place[1] = -1;
+        for (int q = 0; q < 6; ++q) f.q[q] = T.p[q];
+        if (T.kind == MAFM_FX_LJ || T.kind == MAFM_FX_MORSE)
+            for (int q = 0; q < 3; ++q) f.q[3 + q] = T.shift[q];
+        const int* upd = flex_update_order(T.kind);
+        bool any = false;
+        for (int q = 0; q < ar; ++q) {
+            const int r = upd[q], i = T.atom[r];
+            if (!summed[i]) continue;
+            any = true;
+            f.slot[r] = row[next[i]++] + 3 * rank[i];
+            if (i == 1) {
+                if (f.place[0] < 0) f.place[0] = L.n_tip++;
+                else f.place[1] = L.n_tip++;
+                if (k < n_ts) {
+                    ++L.tip_ts_slots;
+                    ++L.tip_ts_terms;
+                }
+            }
+        }
+        if (any) L.terms.push_back(f);
+    }
+    for (FxTerm& f : L.terms)
+        for (int q = 0; q < 2; ++q)
+            if (f.place[q] < 0) f.place[q] = L.n_tip;
+    return L;
 }
 
 mafm_status mafm_scan_flexible(mafm_ctx* c, const mafm_flex_desc* s, const mafm_scan_desc* d,
@@ -1298,42 +1378,12 @@ mafm_status mafm_scan_flexible(mafm_ctx* c, const mafm_flex_desc* s, const mafm_
         if (t >= n_ts && flex_tip_surface(T))
             return fail(c, MAFM_ERR_INVALID, "term %d is a tip-surface term after the first non-tip-surface term", t);
     }
-    // terms acting on a free atom, their result slots, and each free atom's slots in list order
-    // the terms acting on a free atom (in list order, each with its first
-    // result slot), each free atom's slots in list order, the tip's terms
-    std::vector<mafm_flex_term> eval;
-    std::vector<int32_t> csr_off(n + 1, 0), csr, tip_eval;
-    int n_slots = 0, ts_slots = 0, n_ts_eval = 0;
-    std::vector<std::vector<int32_t>> per_atom(n);
-    for (int t = 0; t < s->n_terms; ++t) {
-        const mafm_flex_term& T = s->terms[t];
-        const int ar = flex_arity(T.kind);
-        bool any_free = false;
-        for (int r = 0; r < ar; ++r) any_free |= s->fixed[T.atom[r]] != 1;
-        if (!any_free) continue;
-        const int k = (int)eval.size();
-        eval.push_back(T);
-        eval.back().reserved = n_slots;
-        const int* order = flex_update_order(T.kind);
-        for (int q = 0; q < ar; ++q) {
-            const int r = order[q];
-            if (s->fixed[T.atom[r]] != 1) per_atom[T.atom[r]].push_back(n_slots + r);
-            if (T.atom[r] == 1) tip_eval.push_back(k);   // energies_[1] += e
-        }
-        n_slots += ar;
-        if (t < n_ts) {
-            ts_slots = n_slots;
-            n_ts_eval = k + 1;
-        }
-    }
-    for (int i = 0; i < n; ++i) {
-        csr_off[i + 1] = csr_off[i] + (int32_t)per_atom[i].size();
-        csr.insert(csr.end(), per_atom[i].begin(), per_atom[i].end());
-    }
-    const int n_eval = (int)eval.size();
-    int tip_ts_slots = 0, tip_ts_terms = 0;
-    for (int32_t sl : per_atom[1]) tip_ts_slots += sl < ts_slots;
-    for (int32_t k : tip_eval) tip_ts_terms += k < n_ts_eval;
+    // the terms acting on a free atom; fixed atoms' forces are never read
+    std::vector<char> summed(n);
+    for (int i = 0; i < n; ++i) summed[i] = s->fixed[i] != 1;
+    const FlexList L = flex_list(n, s->n_terms, s->terms, n_ts, s->fixed, summed);
+    const int n_eval = (int)L.terms.size();
+    const int n_ts_eval = n_ts;       // each acts on the tip, which is free
     const size_t n_rec = (size_t)n_cols * d->nz;
 
     HIPCHK(c, hipSetDevice(c->device));
@@ -1343,21 +1393,16 @@ mafm_status mafm_scan_flexible(mafm_ctx* c, const mafm_flex_desc* s, const mafm_
     c->n_records = 0;
     c->last_flex = false;
     c->fx_state_atoms = c->fx_state_heights = 0;
-    std::vector<int32_t> ints;
-    ints.reserve((n + 1) + csr.size() + tip_eval.size() + n);
-    ints.insert(ints.end(), csr_off.begin(), csr_off.end());
-    ints.insert(ints.end(), csr.begin(), csr.end());
-    ints.insert(ints.end(), tip_eval.begin(), tip_eval.end());
-    ints.insert(ints.end(), s->fixed, s->fixed + n);
+    const std::vector<int32_t>& ints = L.idx;
 
     FlexArgs a;
     memset(&a, 0, sizeof a);
-    a.n_atoms = n; a.n_eval = n_eval; a.n_ts = n_ts_eval;
-    a.n_slots = n_slots; a.ts_slots = ts_slots;
-    a.n_csr = (int32_t)csr.size();
-    a.n_tip = (int32_t)tip_eval.size();
-    a.tip_ts_slots = tip_ts_slots;
-    a.tip_ts_terms = tip_ts_terms;
+    a.n_atoms = n;
+    a.n_slots = L.n_slots;
+    a.n_tip = L.n_tip;
+    a.tip_ts_slots = L.tip_ts_slots;
+    a.tip_ts_terms = L.tip_ts_terms;
+    a.tip_rank = L.tip_rank;
     a.nx = d->nx; a.ny = d->ny; a.nz = d->nz;
     a.dx = d->dx; a.dy = d->dy; a.dz = d->dz; a.zhigh = d->zhigh;
     a.minimiser = d->minimiser; a.integrator = d->integrator; a.minterm = d->minterm;
@@ -1368,7 +1413,6 @@ mafm_status mafm_scan_flexible(mafm_ctx* c, const mafm_flex_desc* s, const mafm_
     if (a.tip_pbc) inv3(a.cell, a.cell_inv);
     memcpy(a.offset, s->offset, sizeof a.offset);
     a.tip_dummy_d = s->tip_dummy_d;
-    const bool rk4 = d->minimiser == MAFM_MIN_FIRE && d->integrator == MAFM_INT_RK4;
     // the column state in LDS when one workgroup may hold it (gfx950: up to
     // 160 KiB), as many columns per CU as its LDS holds (up to 8)
     const size_t block_bytes = flex_block_lds(a) + 64;
@@ -1379,23 +1423,19 @@ mafm_status mafm_scan_flexible(mafm_ctx* c, const mafm_flex_desc* s, const mafm_
     int per_cu = 8 / waves;
     if (in_lds) per_cu = (int)std::max<size_t>(1, std::min<size_t>(per_cu, c->lds_per_cu / block_bytes));
     const int n_blocks = (int)std::min<long>(n_cols, (long)c->cus * per_cu);
-    // the term schedule goes behind the index tables (read once per thread,
-    // not copied to LDS)
-    std::vector<int32_t> sched;
-    const int sched_rounds = flex_schedule(eval, waves, sched);
-    const size_t sched_at = ints.size();
-    ints.insert(ints.end(), sched.begin(), sched.end());
+    std::vector<FxTerm> sched;
+    a.rounds = flex_schedule(L.terms, waves, n / 20.0, sched);
 
-    HIPCHK(c, c->d_fx_terms.reserve(std::max(n_eval, 1)));
+    HIPCHK(c, c->d_fx_terms.reserve(std::max<size_t>(sched.size(), 1)));
     HIPCHK(c, c->d_fx_ints.reserve(ints.size()));
     HIPCHK(c, c->d_fx_pos.reserve(3 * (size_t)n));
     HIPCHK(c, c->d_rec.reserve(n_rec));
     HIPCHK(c, c->d_next.reserve(1));
     if (s->state_column >= 0) HIPCHK(c, c->d_fx_state.reserve((size_t)d->nz * n * 3));
-    if (!in_lds) HIPCHK(c, c->d_fx_work.reserve((size_t)n_blocks * flex_block_doubles(n, n_slots, n_eval, rk4)));
-    if (n_eval > 0)
-        HIPCHK(c, hipMemcpyAsync(c->d_fx_terms.p, eval.data(), n_eval * sizeof(mafm_flex_term),
-                                 hipMemcpyHostToDevice, c->stream));
+    if (!in_lds) HIPCHK(c, c->d_fx_work.reserve((size_t)n_blocks * flex_block_doubles(a)));
+    if (!sched.empty())
+        HIPCHK(c, hipMemcpyAsync(c->d_fx_terms.p, sched.data(), sched.size() * sizeof(FxTerm), hipMemcpyHostToDevice,
+                                 c->stream));
     HIPCHK(c, hipMemcpyAsync(c->d_fx_ints.p, ints.data(), ints.size() * sizeof(int32_t), hipMemcpyHostToDevice,
                              c->stream));
     HIPCHK(c, hipMemcpyAsync(c->d_fx_pos.p, s->positions, 3 * (size_t)n * sizeof(double), hipMemcpyHostToDevice,
@@ -1405,8 +1445,6 @@ mafm_status mafm_scan_flexible(mafm_ctx* c, const mafm_flex_desc* s, const mafm_
 
     a.terms = c->d_fx_terms.p;
     a.idx = c->d_fx_ints.p;
-    a.sched = sched_rounds > 0 ? c->d_fx_ints.p + sched_at : nullptr;
-    a.sched_rounds = sched_rounds;
     a.pos0 = c->d_fx_pos.p;
     a.rec = c->d_rec.p;
     a.next_col = c->d_next.p;
@@ -1438,7 +1476,7 @@ mafm_status mafm_scan_flexible(mafm_ctx* c, const mafm_flex_desc* s, const mafm_
         stats->unconverged = counters[1];
         const int64_t evals = d->minimiser == MAFM_MIN_SD ? 1 : (d->integrator == 1 ? 2 : (d->integrator == 2 ? 4 : 1));
         // term evaluations: every evaluated term per integrator stage, plus the tip-surface terms of each output
-        stats->pair_evals = counters[0] * evals * n_eval + (int64_t)n_rec * a.n_ts;
+        stats->pair_evals = counters[0] * evals * n_eval + (int64_t)n_rec * n_ts_eval;
         stats->lanes_per_pixel = 64 * waves;
         stats->grid_blocks = n_blocks;
         stats->block_threads = 64 * waves;
@@ -1470,45 +1508,21 @@ static mafm_status system_op(mafm_ctx* c, const mafm_interaction_list* L, int op
         if (o->integrator < 0 || o->integrator > 2) return fail(c, MAFM_ERR_INVALID, "integrator");
         if (o->minterm < 0 || o->minterm > 2) return fail(c, MAFM_ERR_INVALID, "minterm");
     }
-    std::vector<mafm_flex_term> terms(L->terms, L->terms + L->n_terms);
-    std::vector<std::vector<int32_t>> fslots(n), eterms(n);
-    int n_slots = 0;
     for (int k = 0; k < L->n_terms; ++k) {
-        mafm_flex_term& T = terms[k];
+        const mafm_flex_term& T = L->terms[k];
         const int ar = flex_arity(T.kind);
         if (ar == 0) return fail(c, MAFM_ERR_INVALID, "term %d: unknown kind %d", k, T.kind);
         for (int r = 0; r < ar; ++r)
             if (T.atom[r] < 0 || T.atom[r] >= n)
                 return fail(c, MAFM_ERR_INVALID, "term %d: atom %d outside 0..%d", k, T.atom[r], n - 1);
-        T.reserved = n_slots;
-        const int* order = flex_update_order(T.kind);
-        for (int q = 0; q < ar; ++q) {
-            const int r = order[q];
-            fslots[T.atom[r]].push_back(n_slots + r);
-            eterms[T.atom[r]].push_back(k);
-        }
-        n_slots += ar;
     }
-    std::vector<int32_t> ints;
-    auto csr = [&](const std::vector<std::vector<int32_t>>& lists) {
-        size_t start = ints.size(), total = 0;
-        ints.resize(start + n + 1);
-        for (int i = 0; i < n; ++i) {
-            ints[start + i] = (int32_t)total;
-            total += lists[i].size();
-        }
-        ints[start + n] = (int32_t)total;
-        for (const auto& l : lists) ints.insert(ints.end(), l.begin(), l.end());
-        return (int32_t)total;
-    };
+    const FlexList list = flex_list(n, L->n_terms, L->terms, 0, L->fixed, std::vector<char>(n, 1));
+    const std::vector<int32_t>& ints = list.idx;
     SysArgs a;
     memset(&a, 0, sizeof a);
-    a.n_fcsr = csr(fslots);
-    a.n_ecsr = csr(eterms);
-    ints.insert(ints.end(), L->fixed, L->fixed + n);
     a.n_atoms = n;
-    a.n_terms = L->n_terms;
-    a.n_slots = n_slots;
+    a.n_slots = list.n_slots;
+    a.n_tip = list.n_tip;
     a.op = op;
     a.integrator = integrator;
     a.dt = dt;
@@ -1527,10 +1541,12 @@ static mafm_status system_op(mafm_ctx* c, const mafm_interaction_list* L, int op
     const int waves = std::max(L->n_terms, n) > 128 ? 4 : (std::max(L->n_terms, n) > 64 ? 2 : 1);
     const size_t n3 = (size_t)n_states * n * 3, n1 = (size_t)n_states * n;
     const int64_t blocks = std::min<int64_t>(n_states, 1 << 20);
-    const size_t nd = (sys_block_bytes(a) - ints.size() * sizeof(int32_t)) / sizeof(double);
+    const size_t nd = sys_block_doubles(a);
+    std::vector<FxTerm> sched;
+    a.rounds = flex_schedule(list.terms, waves, op == SYS_MINIMISE ? n / 20.0 : 0.0, sched);
 
     HIPCHK(c, hipSetDevice(c->device));
-    HIPCHK(c, c->d_fx_terms.reserve(std::max(L->n_terms, 1)));
+    HIPCHK(c, c->d_fx_terms.reserve(std::max<size_t>(sched.size(), 1)));
     HIPCHK(c, c->d_fx_ints.reserve(ints.size()));
     HIPCHK(c, c->d_sys.reserve(3 * n3 + n1 + (n_states + 1) / 2 + 1));
     if (!in_lds) HIPCHK(c, c->d_fx_work.reserve((size_t)blocks * nd));
@@ -1539,9 +1555,9 @@ static mafm_status system_op(mafm_ctx* c, const mafm_interaction_list* L, int op
     double* d_frc = d_vel + n3;
     double* d_ener = d_frc + n3;
     int32_t* d_steps = reinterpret_cast<int32_t*>(d_ener + n1);
-    if (L->n_terms > 0)
-        HIPCHK(c, hipMemcpyAsync(c->d_fx_terms.p, terms.data(), terms.size() * sizeof(mafm_flex_term),
-                                 hipMemcpyHostToDevice, c->stream));
+    if (!sched.empty())
+        HIPCHK(c, hipMemcpyAsync(c->d_fx_terms.p, sched.data(), sched.size() * sizeof(FxTerm), hipMemcpyHostToDevice,
+                                 c->stream));
     HIPCHK(c, hipMemcpyAsync(c->d_fx_ints.p, ints.data(), ints.size() * sizeof(int32_t), hipMemcpyHostToDevice,
                              c->stream));
     HIPCHK(c, hipMemcpyAsync(d_pos, pos, n3 * sizeof(double), hipMemcpyHostToDevice, c->stream));

@@ -6,34 +6,37 @@
 
 namespace mafm {
 
-// Every term is evaluated once per integrator stage into result slots, one
-// slot {fx, fy, fz} per atom the term acts on, holding the signed force that
-// atom receives (the reference's `forces[i] -= f` is `+= -f`, the same
-// rounding), plus the term's energy.  Each free atom then sums its slots in
-// the interaction list's order; the tip sums the energies of its terms.
+// One interaction as the kernels read it.  Every term is evaluated once per
+// integrator stage into result slots {fx, fy, fz}, one per atom it acts on,
+// holding the signed force that atom receives (the reference's `forces[i] -= f`
+// is `+= -f`, the same rounding).  An atom's slots are numbered in the
+// interaction list's order, the order its force is summed in; slot q of the atom
+// of rank k (atoms by falling number of slots) has its components at row[q] + 3 k.
+struct FxTerm {
+    int32_t kind;                     // MAFM_FX_*; -1: nothing to evaluate
+    int32_t atom[4];
+    int32_t slot[4];                  // place of each atom's result slot; 3 n_slots: not read
+    int32_t place[2];                 // place of its energy in the tip's list; n_tip: not read
+    int32_t pad;
+    double q[6];                      // pair terms: p0, p1, p2, shift x, y, z; else mafm_flex_term::p
+};
+
+// The term records lie in schedule order: thread l of the block takes record
+// r * block threads + l in rounds r < rounds.  The schedule only places the
+// work; the slots are summed in list order.
 struct FlexArgs {
-    int32_t n_atoms, n_eval, n_ts;    // eval entries [0, n_ts) are the tip-surface terms
-    int32_t n_slots, ts_slots;        // slots [0, ts_slots) belong to the tip-surface terms
+    int32_t n_atoms, n_slots, n_tip;  // n_tip: terms acting on the tip (an energy place each)
+    int32_t tip_ts_slots, tip_ts_terms;   // the tip's first slots / terms, from tip-surface terms
     int32_t nx, ny, nz;
     double dx, dy, dz, zhigh;
     int32_t minimiser, integrator, minterm, maxsteps;
     double etol, ftol, dt;
-    // the terms that act on a free atom, in list order, each with its first
-    // result slot in `reserved`
-    const mafm_flex_term* terms;
-    // index tables, back to back: csr_off (n_atoms + 1, empty ranges for fixed
-    // atoms), csr (n_csr: the result slots of each free atom in list order),
-    // tip_eval (n_tip: the terms acting on the tip, in list order), fixed (n_atoms)
+    const FxTerm* terms;
+    int32_t rounds;
+    // index tables, back to back: slots of each rank (none for fixed atoms), its
+    // atom, fixed flags by atom (n_atoms each), the rows' places (and eight more)
     const int32_t* idx;
-    int32_t n_csr, n_tip;
-    int32_t tip_ts_slots, tip_ts_terms;   // the tip's slots / terms from tip-surface terms
-    // which terms each thread evaluates in one integrator stage: thread l of
-    // the block takes sched[r * block threads + l] (-1: none) in rounds
-    // r < sched_rounds; NULL: terms l, l + T, ...
-    // The schedule only places the work: every term still writes its own
-    // result slots, which are summed in list order.
-    const int32_t* sched;
-    int32_t sched_rounds;
+    int32_t tip_rank;
     const double* pos0;               // n_atoms x 3
     int32_t tip_pbc;
     int32_t state_col;                // column whose positions are kept per height, -1 none
@@ -51,17 +54,13 @@ struct FlexArgs {
 // minimisation from the given state.
 enum { SYS_EVAL = 0, SYS_STEP = 1, SYS_MINIMISE = 2 };
 struct SysArgs {
-    int32_t n_atoms, n_terms, n_slots, op;
+    int32_t n_atoms, n_slots, n_tip, op;
     int32_t minimiser, integrator, minterm, maxsteps;
     double etol, ftol, dt;
     int64_t n_states;
-    // every term, in list order, its first result slot in `reserved`
-    const mafm_flex_term* terms;
-    // back to back: f_off (n_atoms + 1), f_csr (n_fcsr: each atom's result
-    // slots in list order), e_off (n_atoms + 1), e_csr (n_ecsr: each atom's
-    // terms in list order, for its energy), fixed (n_atoms)
-    const int32_t* idx;
-    int32_t n_fcsr, n_ecsr;
+    const FxTerm* terms;              // as FlexArgs; every atom's roles have a slot
+    int32_t rounds;
+    const int32_t* idx;               // as FlexArgs
     double* pos;       // n_states x n_atoms x 3, in and out
     double* vel;       // n_states x n_atoms x 3, in and out (step, minimise)
     double* frc;       // n_states x n_atoms x 3: in (eval and the Euler step add to it), out
@@ -69,12 +68,13 @@ struct SysArgs {
     int32_t* steps;    // n_states (minimise)
     double* work;      // per-block state when it does not fit LDS
 };
-size_t sys_block_bytes(const SysArgs& a);
+size_t sys_block_doubles(const SysArgs& a);
+size_t sys_block_bytes(const SysArgs& a);   // with the index tables
 hipError_t launch_system_op(const SysArgs& a, int waves, bool in_lds, hipStream_t st);
 
 // Doubles of per-column state one block keeps (positions, integrator
 // stages, velocities, forces, term results).
-size_t flex_block_doubles(int n_atoms, int n_slots, int n_eval, bool rk4);
+size_t flex_block_doubles(const FlexArgs& a);
 // LDS bytes of one block when the state lives there (state + index tables).
 size_t flex_block_lds(const FlexArgs& a);
 // waves: wavefronts per workgroup (1-4); in_lds: the state lives in LDS (else
