@@ -146,12 +146,10 @@ class ScanModel:
     def _system(self, es6, es12, qq, pos) -> abi.SystemDesc:
         n = len(es6)
         arr = (abi.Site * n)()
-        for i in range(n):
-            arr[i].x, arr[i].y, arr[i].z = (float(v) for v in pos[i])
-            arr[i].vdw = abi.VDW_LJ
-            arr[i].has_coulomb = int(self.has_coulomb[i])
-            arr[i].p0, arr[i].p1, arr[i].p2 = float(es6[i]), float(es12[i]), 0.0
-            arr[i].qq = float(qq[i])
+        sites = np.frombuffer(arr, dtype=np.dtype(abi.Site))
+        for k, v in dict(x=pos[:, 0], y=pos[:, 1], z=pos[:, 2], vdw=abi.VDW_LJ, has_coulomb=self.has_coulomb,
+                         p0=es6, p1=es12, p2=0.0, qq=qq).items():
+            sites[k] = v
         d = abi.SystemDesc()
         ctypes.pointer(d)[0] = self.desc
         d.n_sites = n
@@ -166,12 +164,22 @@ class ScanModel:
         self.last_records, self.last_stats = rec, stats
         # records report the requested pixel (x, y); with a unit cell the
         # scan ran at its wrapped image, where the tip relaxed
-        x, y = rec["x"].copy(), rec["y"].copy()
+        # (a column's heights share their pixel: one wrap each)
+        nz = self.shape[2]
+        x, y = rec["x"][::nz], rec["y"][::nz]
         if self.desc.tip_pbc:
             x, y = wrap_dummy_xy(self.desc.cell, self.desc.offset, x, y)
-        dummy = np.stack([x, y, rec["z"]], 1)
-        tip = dummy + np.stack([rec["rx"], rec["ry"], rec["rz"]], 1)
-        return rec["fz"].copy(), tip, dummy
+        # torch gathers the fields with every core; numpy's strided copies of
+        # half a million records took 11 ms of a 39 ms step on one
+        raw = torch.from_numpy(rec.view(np.float64).reshape(len(rec), rec.dtype.itemsize // 8))
+        field = {k: rec.dtype.fields[k][1] // 8 for k in ("z", "fz", "rx")}
+        dummy = torch.empty(len(rec), 3, dtype=torch.float64)
+        cols = dummy.view(-1, nz, 3)
+        cols[:, :, 0] = torch.from_numpy(np.ascontiguousarray(x))[:, None]
+        cols[:, :, 1] = torch.from_numpy(np.ascontiguousarray(y))[:, None]
+        dummy[:, 2] = raw[:, field["z"]]
+        tip = dummy + raw[:, field["rx"]:field["rx"] + 3]
+        return raw[:, field["fz"]].contiguous().numpy(), tip.numpy(), dummy.numpy()
 
     def adjoint_np(self, es6, es12, qq, pos, tip, dummy, g):
         self.ctx.set_systems([self._system(es6, es12, qq, pos)])

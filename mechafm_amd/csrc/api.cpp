@@ -15,6 +15,7 @@
 #include <thread>
 #include <vector>
 
+#include "host_link.hpp"
 #include "../../include/mafm.h"
 #include "ctx_ref.hpp"
 #include "device_common.hpp"
@@ -117,6 +118,17 @@ struct DevBuf {
         p = nullptr;
         cap = 0;
     }
+    T* take() {   // the memory, now the caller's
+        T* q = p;
+        p = nullptr;
+        cap = 0;
+        return q;
+    }
+    void give(T* q, size_t n) {   // memory of n elements, now this buffer's
+        release();
+        p = q;
+        cap = n;
+    }
 };
 
 // Pinned, coherent host memory mapped into the device's address space: the
@@ -186,6 +198,10 @@ struct mafm_ctx {
     DevBuf<int32_t> d_order;
     DevBuf<int64_t> d_counters;
     DevBuf<double> d_tmp;
+    DevBuf<double> d_work;         // workspace of one call (transforms, adjoint, images): see Work
+    DevBuf<double4> spare64;       // the last freed grid's buffers, for the next grid
+    DevBuf<float4> spare32;
+    HostLink link;                 // results to pageable arrays
     DevBuf<float4> d_margins;      // per-position decision margins (MAFM_SCAN_MARGINS)
     // streamed scans (mafm_scan_host): records and per-column flags in pinned host memory
     HostBuf<DevRecord> h_rec;
@@ -232,6 +248,25 @@ static mafm_status fail(mafm_ctx* c, mafm_status s, const char* fmt, ...) {
             return fail(ctx, MAFM_ERR_HIP, "%s failed: %s", #expr, hipGetErrorString(e_));        \
     } while (0)
 
+// Device memory a context keeps for the next call beyond its tables and
+// records: the workspace and one freed grid, each up to this size (hipFree waits
+// for the device and hipMalloc maps pages: 2 ms a potential of 2 M points).
+static constexpr size_t KEPT_BYTES = (size_t)512 << 20;
+
+// The context's workspace for one call, which ends with the stream idle; a
+// large one is given back then.
+struct Work {
+    mafm_ctx* c;
+    explicit Work(mafm_ctx* ctx) : c(ctx) {}
+    Work(const Work&) = delete;
+    Work& operator=(const Work&) = delete;
+    ~Work() {
+        if (c->d_work.cap * sizeof(double) > KEPT_BYTES) c->d_work.release();
+    }
+    hipError_t reserve(size_t doubles) { return c->d_work.reserve(doubles); }
+    double* p() const { return c->d_work.p; }
+};
+
 static mafm_status sync_grids(mafm_ctx* c) {
     std::vector<DevGrid> dg(std::max<size_t>(c->grids.size(), 1));
     for (size_t k = 0; k < c->grids.size(); ++k) {
@@ -267,8 +302,14 @@ static mafm_status new_grid(mafm_ctx* c, const mafm_grid_desc* g, HostGrid& h) {
     if (h.orthogonal)   // exact reciprocals of the spacings (the fast lookups multiply by them)
         for (int d = 0; d < 3; ++d) h.inv[4 * d] = 1.0 / h.basis[4 * d];
     size_t np = (size_t)h.n[0] * h.n[1] * h.n[2];
-    HIPCHK(c, hipMalloc(&h.fe64, np * sizeof(double4)));
-    HIPCHK(c, hipMalloc(&h.fe32, np * sizeof(float4)));
+    // a grid as large as the one freed last (a scan's grid rebuilt for new parameters) takes its buffers
+    if (np == c->spare64.cap && np == c->spare32.cap) {
+        h.fe64 = c->spare64.take();
+        h.fe32 = c->spare32.take();
+    } else {
+        HIPCHK(c, hipMalloc(&h.fe64, np * sizeof(double4)));
+        HIPCHK(c, hipMalloc(&h.fe32, np * sizeof(float4)));
+    }
     h.live = true;
     return MAFM_OK;
 }
@@ -784,8 +825,7 @@ mafm_status mafm_grid_download(mafm_ctx* c, int handle, double* fe) {
         return fail(c, MAFM_ERR_INVALID, "grid handle %d is not live", handle);
     const HostGrid& h = c->grids[handle];
     size_t np = (size_t)h.n[0] * h.n[1] * h.n[2];
-    HIPCHK(c, hipMemcpyAsync(fe, h.fe64, np * sizeof(double4), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, c->link.to_host(fe, h.fe64, np * sizeof(double4), c->device, c->stream));
     return MAFM_OK;
 }
 
@@ -840,8 +880,13 @@ mafm_status mafm_grid_free(mafm_ctx* c, int handle) {
             return fail(c, MAFM_ERR_STATE, "grid %d is used by a loaded system", handle);
     HIPCHK(c, hipStreamSynchronize(c->stream));
     HostGrid& h = c->grids[handle];
-    (void)hipFree(h.fe64);
-    (void)hipFree(h.fe32);
+    const size_t np = (size_t)h.n[0] * h.n[1] * h.n[2];
+    c->spare64.give(h.fe64, np);
+    c->spare32.give(h.fe32, np);
+    if (np * (sizeof(double4) + sizeof(float4)) > KEPT_BYTES) {
+        c->spare64.release();
+        c->spare32.release();
+    }
     h = HostGrid();
     return sync_grids(c);
 }
@@ -890,17 +935,18 @@ mafm_status mafm_grid_build(mafm_ctx* c, const mafm_system_desc* sys, const mafm
     s = new_grid(c, g, h);
     if (s != MAFM_OK) return s;
     if (!h.orthogonal) return fail(c, MAFM_ERR_INVALID, "grid build expects a diagonal spacing basis");
-    DevBuf<DevMol> dm;
-    DevBuf<Site64> dr;
-    HIPCHK(c, dm.reserve(1));
-    HIPCHK(c, dr.reserve(ref.size()));
-    HIPCHK(c, hipMemcpyAsync(dm.p, mols.data(), sizeof(DevMol), hipMemcpyHostToDevice, c->stream));
+    static_assert(sizeof(Site64) % sizeof(double) == 0 && alignof(DevMol) <= alignof(double), "table layout");
+    Work work(c);
+    HIPCHK(c, work.reserve((ref.size() * sizeof(Site64) + sizeof(DevMol)) / sizeof(double) + 1));
+    Site64* dr = reinterpret_cast<Site64*>(work.p());
+    DevMol* dm = reinterpret_cast<DevMol*>(dr + ref.size());
+    HIPCHK(c, hipMemcpyAsync(dm, mols.data(), sizeof(DevMol), hipMemcpyHostToDevice, c->stream));
     if (!ref.empty())
-        HIPCHK(c, hipMemcpyAsync(dr.p, ref.data(), ref.size() * sizeof(Site64), hipMemcpyHostToDevice, c->stream));
+        HIPCHK(c, hipMemcpyAsync(dr, ref.data(), ref.size() * sizeof(Site64), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemsetAsync(c->d_counters.p, 0, 8 * sizeof(int64_t), c->stream));
     ScanArgs a = base_args(c);
-    a.mols = dm.p;
-    a.sites_ref = dr.p;
+    a.mols = dm;
+    a.sites_ref = dr;
     a.n_mols = 1;
     const double sp[3] = {h.basis[0], h.basis[4], h.basis[8]};
     HIPCHK(c, launch_grid_build(a, 0, h.n, sp, h.offset, h.fe64, c->stream));
@@ -909,8 +955,6 @@ mafm_status mafm_grid_build(mafm_ctx* c, const mafm_system_desc* sys, const mafm
     int64_t counters[8];
     HIPCHK(c, hipMemcpyAsync(counters, c->d_counters.p, sizeof counters, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    dm.release();
-    dr.release();
     if (counters[3] != 0) return fail(c, MAFM_ERR_OUT_OF_GRID, "potential-grid lookup left the grid during grid build");
     *handle = store_grid(c, h);
     guard.kept = true;
@@ -1623,8 +1667,7 @@ mafm_status mafm_margins(mafm_ctx* c, size_t first, size_t count, float* out) {
         return fail(c, MAFM_ERR_INVALID, "margins [%zu, %zu) beyond the %zu of the last scan", first, first + count,
                     c->n_records);
     if (count == 0) return MAFM_OK;
-    HIPCHK(c, hipMemcpyAsync(out, c->d_margins.p + first, count * sizeof(float4), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, c->link.to_host(out, c->d_margins.p + first, count * sizeof(float4), c->device, c->stream));
     return MAFM_OK;
 }
 
@@ -1649,12 +1692,12 @@ mafm_status mafm_delta_f(mafm_ctx* c, int system, const mafm_deltaf_desc* d, dou
     if (w.n_images == 0) return fail(c, MAFM_ERR_INVALID, "%d heights do not fill a %d-height window", s.nz, w.n_weights);
     HIPCHK(c, hipSetDevice(c->device));
     const size_t n = (size_t)w.n_images * s.nx * s.ny;
-    DevBuf<double> out;
-    HIPCHK(c, out.reserve(n));
+    Work work(c);
+    HIPCHK(c, work.reserve(n));
+    double* out = work.p();
     const DevRecord* rec = c->d_rec.p + (c->last_flex ? 0 : c->mols[system].rec_off);
-    HIPCHK(c, launch_delta_f(rec, w, s.nx, s.ny, s.nz, d->fz_from_text != 0, out.p, c->stream));
-    HIPCHK(c, hipMemcpyAsync(df, out.p, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, launch_delta_f(rec, w, s.nx, s.ny, s.nz, d->fz_from_text != 0, out, c->stream));
+    HIPCHK(c, c->link.to_host(df, out, n * sizeof(double), c->device, c->stream));
     if (z_low) memcpy(z_low, zl.data(), zl.size() * sizeof(double));
     return MAFM_OK;
 }
@@ -1666,8 +1709,7 @@ mafm_status mafm_records(mafm_ctx* c, size_t first, size_t count, mafm_record* o
                     c->n_records);
     static_assert(sizeof(mafm_record) == sizeof(DevRecord), "record layout");
     if (count == 0) return MAFM_OK;
-    HIPCHK(c, hipMemcpyAsync(out, c->d_rec.p + first, count * sizeof(DevRecord), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, c->link.to_host(out, c->d_rec.p + first, count * sizeof(DevRecord), c->device, c->stream));
     return MAFM_OK;
 }
 
@@ -1727,15 +1769,14 @@ mafm_status mafm_fft3d(mafm_ctx* c, const int32_t n[3], int inverse, const doubl
     const double2* tw[3];
     for (int a = 0; a < 3; ++a)
         if ((s = twiddles_for(c, n[a], &tw[a])) != MAFM_OK) return s;
-    DevBuf<double2> d;
-    HIPCHK(c, d.reserve(N));
-    HIPCHK(c, hipMemcpyAsync(d.p, in, N * sizeof(double2), hipMemcpyHostToDevice, c->stream));
+    Work work(c);
+    HIPCHK(c, work.reserve(2 * (size_t)N));
+    double2* d = reinterpret_cast<double2*>(work.p());
+    HIPCHK(c, hipMemcpyAsync(d, in, N * sizeof(double2), hipMemcpyHostToDevice, c->stream));
     int nn[3] = {n[0], n[1], n[2]};
-    HIPCHK(c, fft3d_device(d.p, nn, tw, inverse != 0, c->stream));
-    if (inverse) HIPCHK(c, launch_scale2(d.p, 1.0 / (double)N, N, c->stream));
-    HIPCHK(c, hipMemcpyAsync(out, d.p, N * sizeof(double2), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    d.release();
+    HIPCHK(c, fft3d_device(d, nn, tw, inverse != 0, c->stream));
+    if (inverse) HIPCHK(c, launch_scale2(d, 1.0 / (double)N, N, c->stream));
+    HIPCHK(c, c->link.to_host(out, d, N * sizeof(double2), c->device, c->stream));
     return MAFM_OK;
 }
 
@@ -1777,22 +1818,22 @@ mafm_status mafm_potential_grid(mafm_ctx* c, const mafm_potential_desc* pd, int*
     const double2* tw[3];
     for (int a = 0; a < 3; ++a)
         if ((s = twiddles_for(c, n[a], &tw[a])) != MAFM_OK) return s;
-    DevBuf<double2> pot, rho, tmp;
-    DevBuf<double> real;
-    HIPCHK(c, pot.reserve(N));
-    HIPCHK(c, rho.reserve(N));
-    HIPCHK(c, tmp.reserve(N));
-    HIPCHK(c, real.reserve(N));
+    Work work(c);
+    HIPCHK(c, work.reserve(7 * (size_t)N));
+    double2* pot = reinterpret_cast<double2*>(work.p());
+    double2* rho = pot + N;
+    double2* tmp = rho + N;
+    double* real = work.p() + 6 * N;
     HIPCHK(c, c->d_flag.reserve(1));
     HIPCHK(c, hipMemsetAsync(c->d_flag.p, 0, sizeof(int), c->stream));
-    HIPCHK(c, hipMemcpyAsync(real.p, pd->potential, N * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(real, pd->potential, N * sizeof(double), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-    HIPCHK(c, launch_real_to_complex(real.p, pot.p, N, c->stream));
-    HIPCHK(c, launch_zero2(rho.p, N, c->stream));
-    HIPCHK(c, launch_gauss_tip(rho.p, n, cut, ortho, B, pd->tip_charge * norm, w2, c->stream));
-    HIPCHK(c, fft3d_device(pot.p, n, tw, false, c->stream));
-    HIPCHK(c, fft3d_device(rho.p, n, tw, false, c->stream));
-    HIPCHK(c, launch_mul_vol(pot.p, rho.p, vol, N, c->stream));   // pot = E_k
+    HIPCHK(c, launch_real_to_complex(real, pot, N, c->stream));
+    HIPCHK(c, launch_zero2(rho, N, c->stream));
+    HIPCHK(c, launch_gauss_tip(rho, n, cut, ortho, B, pd->tip_charge * norm, w2, c->stream));
+    HIPCHK(c, fft3d_device(pot, n, tw, false, c->stream));
+    HIPCHK(c, fft3d_device(rho, n, tw, false, c->stream));
+    HIPCHK(c, launch_mul_vol(pot, rho, vol, N, c->stream));   // pot = E_k
     HostGrid h;
     mafm_grid_desc gd{};
     for (int a = 0; a < 3; ++a) {
@@ -1806,23 +1847,19 @@ mafm_status mafm_potential_grid(mafm_ctx* c, const mafm_potential_desc* pd, int*
     if (s != MAFM_OK) return s;
     double* fe = reinterpret_cast<double*>(h.fe64);
     const double inv_n = 1.0 / (double)N;
-    HIPCHK(c, hipMemcpyAsync(tmp.p, pot.p, N * sizeof(double2), hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(c, fft3d_device(tmp.p, n, tw, true, c->stream));
-    HIPCHK(c, launch_extract(tmp.p, fe, 3, inv_n, N, c->d_flag.p, c->stream));
+    HIPCHK(c, hipMemcpyAsync(tmp, pot, N * sizeof(double2), hipMemcpyDeviceToDevice, c->stream));
+    HIPCHK(c, fft3d_device(tmp, n, tw, true, c->stream));
+    HIPCHK(c, launch_extract(tmp, fe, 3, inv_n, N, c->d_flag.p, c->stream));
     for (int comp = 0; comp < 3; ++comp) {
-        HIPCHK(c, launch_spectral_grad(pot.p, tmp.p, n, comp, kb, c->stream));
-        HIPCHK(c, fft3d_device(tmp.p, n, tw, true, c->stream));
-        HIPCHK(c, launch_extract(tmp.p, fe, comp, inv_n, N, c->d_flag.p, c->stream));
+        HIPCHK(c, launch_spectral_grad(pot, tmp, n, comp, kb, c->stream));
+        HIPCHK(c, fft3d_device(tmp, n, tw, true, c->stream));
+        HIPCHK(c, launch_extract(tmp, fe, comp, inv_n, N, c->d_flag.p, c->stream));
     }
     HIPCHK(c, launch_to_f32(h.fe64, h.fe32, N, c->stream));
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     int flag = 0;
     HIPCHK(c, hipMemcpyAsync(&flag, c->d_flag.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    pot.release();
-    rho.release();
-    tmp.release();
-    real.release();
     if (flag) {
         return fail(c, MAFM_ERR_FFT_IMAG, "Imaginary part of inverse FFT exceeded threshold 1.0e-8!");
     }
@@ -1844,9 +1881,9 @@ mafm_status mafm_adjoint(mafm_ctx* c, int system, const mafm_adjoint_desc* d, ma
     const int ns = m.n_sites;
     if (ns > 0 && (!o->d_es6 || !o->d_es12 || !o->d_qq || !o->d_pos)) return fail(c, MAFM_ERR_INVALID, "adjoint outputs");
     HIPCHK(c, hipSetDevice(c->device));
-    DevBuf<double> buf;
-    HIPCHK(c, buf.reserve((size_t)10 * n + 6 * (size_t)ns + 1));
-    double* tip = buf.p;
+    Work work(c);
+    HIPCHK(c, work.reserve((size_t)10 * n + 6 * (size_t)ns + 1));
+    double* tip = work.p();
     double* dummy = tip + 3 * n;
     double* g = dummy + 3 * n;
     double* v = g + n;
@@ -1867,7 +1904,6 @@ mafm_status mafm_adjoint(mafm_ctx* c, int system, const mafm_adjoint_desc* d, ma
     if (ns) HIPCHK(c, hipMemcpyAsync(h.data(), out6, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipMemcpyAsync(&singular, c->d_flag.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    buf.release();
     for (int i = 0; i < ns; ++i) {
         o->d_es6[i] = h[6 * i];
         o->d_es12[i] = h[6 * i + 1];
