@@ -24,6 +24,8 @@
 namespace mafm {
 hipError_t launch_scan_plain(const ScanArgs& a, hipStream_t st);
 hipError_t launch_eval_plain(const ScanArgs& a, int mol, long n, const double* pos, double* out, hipStream_t st);
+hipError_t launch_eval_split(const ScanArgs& a, int mol, int n, int lanes, const double* pos, double* out,
+                             int* off_grid, hipStream_t st);
 hipError_t launch_grid_interp(const ScanArgs& a, int grid, long n, const double* pos, double* out, hipStream_t st);
 size_t valu_calibration_doubles();
 hipError_t launch_valu_calibration(int kind, int n, double* out, int64_t* wave_insts, hipStream_t st);
@@ -201,6 +203,7 @@ struct mafm_ctx {
     DevBuf<double> d_work;         // workspace of one call (transforms, adjoint, images): see Work
     DevBuf<double4> spare64;       // the last freed grid's buffers, for the next grid
     DevBuf<float4> spare32;
+    HostBuf<double> h_eval;        // points and results of a small tip-surface evaluation
     HostLink link;                 // results to pageable arrays
     DevBuf<float4> d_margins;      // per-position decision margins (MAFM_SCAN_MARGINS)
     // streamed scans (mafm_scan_host): records and per-column flags in pinned host memory
@@ -1713,19 +1716,52 @@ mafm_status mafm_records(mafm_ctx* c, size_t first, size_t count, mafm_record* o
     return MAFM_OK;
 }
 
+// Lanes a point of the tip-surface operator: one lane a point leaves the chip
+// idle and walks the sites in series; more lanes pay for the ordered sum.  150
+// sites, us a call (1 / 16 / 64 lanes): one point 102 / 26 / 20, 1000 points 120 /
+// 28 / 24, 10000 points 146 / 92 / 96, 100000 points 463 / 464 / 535, 300000
+// points 1121 / 1192 / 1404.
+static int eval_lanes(const DevMol& m, size_t n) {
+    if (m.force_grid >= 0 || n > 131072) return 1;
+    return n <= 4096 && m.n_sites > 16 ? 64 : 16;
+}
+
+// Up to this many points the kernel reads them from and writes to pinned host
+// memory: no copies, no counters to clear (4096 points 34 us, by copies 71).
+// The memory is a once-paid 0.3 ms at this size, 0.9 at four times it.
+static constexpr size_t EVAL_MAPPED = 8192;
+
 mafm_status mafm_eval_tip_surface(mafm_ctx* c, int system, size_t n, const double* pos, double* fe) {
     if (!c || (n && (!pos || !fe))) return MAFM_ERR_INVALID;
     if (!c->have_systems) return fail(c, MAFM_ERR_STATE, "eval before mafm_set_systems");
     if (system < 0 || system >= (int)c->mols.size()) return fail(c, MAFM_ERR_INVALID, "system %d", system);
     if (n == 0) return MAFM_OK;
     HIPCHK(c, hipSetDevice(c->device));
+    const int lanes = eval_lanes(c->mols[system], n);
+    if (lanes > 1 && n <= EVAL_MAPPED) {
+        HIPCHK(c, c->h_eval.reserve(7 * std::max<size_t>(n, 1024) + 1));
+        double* io = c->h_eval.p;
+        double* dio = c->h_eval.dp;
+        memcpy(io, pos, 3 * n * sizeof(double));
+        int* off_grid = reinterpret_cast<int*>(io + 7 * n);
+        *off_grid = 0;
+        HIPCHK(c, launch_eval_split(base_args(c), system, (int)n, lanes, dio, dio + 3 * n,
+                                    reinterpret_cast<int*>(dio + 7 * n), c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        memcpy(fe, io + 3 * n, 4 * n * sizeof(double));
+        if (*off_grid) return fail(c, MAFM_ERR_OUT_OF_GRID, "tip position past the force grid");
+        return MAFM_OK;
+    }
     HIPCHK(c, c->d_tmp.reserve(7 * n));
     double* dpos = c->d_tmp.p;
     double* dout = c->d_tmp.p + 3 * n;
     HIPCHK(c, hipMemcpyAsync(dpos, pos, 3 * n * sizeof(double), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemsetAsync(c->d_counters.p, 0, 8 * sizeof(int64_t), c->stream));
     ScanArgs a = base_args(c);
-    HIPCHK(c, launch_eval_plain(a, system, (long)n, dpos, dout, c->stream));
+    if (lanes > 1)   // counters[3] is zero or, one point off the grid, not
+        HIPCHK(c, launch_eval_split(a, system, (int)n, lanes, dpos, dout,
+                                    reinterpret_cast<int*>(c->d_counters.p + 3), c->stream));
+    else HIPCHK(c, launch_eval_plain(a, system, (long)n, dpos, dout, c->stream));
     int64_t counters[8];
     HIPCHK(c, hipMemcpyAsync(fe, dout, 4 * n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipMemcpyAsync(counters, c->d_counters.p, sizeof counters, hipMemcpyDeviceToHost, c->stream));

@@ -64,26 +64,6 @@ __device__ inline V3 cross(V3 a, V3 b) {                                        
     return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
 
-// Quotients by one divisor: the reciprocal's two Newton steps are shared, and
-// each quotient is rounded by the residual step IEEE division ends with (the
-// operations, and so the bits, of the compiler's a / d where it does not
-// rescale its operands, which it does below 2^-970 and near the exponent's
-// ends; div_fixup covers zeros, infinities and NaN).  An angle term has
-// fourteen divisions by two lengths: 11 instructions each become 4.
-struct Divisor {
-    double d, y;
-    __device__ explicit Divisor(double d_) : d(d_) {
-        y = __builtin_amdgcn_rcp(d);
-        y = fma(y, fma(-d, y, 1.0), y);
-        y = fma(y, fma(-d, y, 1.0), y);
-    }
-    __device__ double operator()(double a) const {
-        const double q = a * y;
-        return __builtin_amdgcn_div_fixup(fma(fma(-d, q, a), y, q), d, a);
-    }
-    __device__ V3 operator()(V3 v) const { return {(*this)(v.x), (*this)(v.y), (*this)(v.z)}; }
-};
-
 // A term as a thread holds it: the atoms it acts on, the result slot of each
 // (n_slots: nobody reads it), where the tip's energy list keeps its energy, and
 // its numbers q (pair terms: p0, p1, p2, shift; the others: p).  Packed: 16-bit

@@ -115,14 +115,12 @@ __device__ void eval_tip(Ctx& c, V3 dummy, V3 tip, bool ts_only, V3& F, double& 
             // positions[i2] + pbc_shift, subtracted from the tip (interactions.cpp:16)
             V3 r = {tip.x - (st.x + m.shift[im][0]), tip.y - (st.y + m.shift[im][1]),
                     tip.z - (st.z + m.shift[im][2])};
-            V3 fv; double ev;
-            vdw(st.vdw, st.p0, st.p1, st.p2, r, fv, ev);
-            f.x += fv.x; f.y += fv.y; f.z += fv.z;
-            e += ev;
+            const SiteTerms t = site_terms(st.vdw, st.coul, st.p0, st.p1, st.p2, st.qq, r);
+            f.x += t.f.x; f.y += t.f.y; f.z += t.f.z;
+            e += t.e;
             if (st.coul) {
-                coulomb(st.qq, r, fv, ev);
-                f.x += fv.x; f.y += fv.y; f.z += fv.z;
-                e += ev;
+                f.x += t.fc.x; f.y += t.fc.y; f.z += t.fc.z;
+                e += t.ec;
             }
         }
         if (m.potential_grid >= 0) {
@@ -332,6 +330,69 @@ __global__ void __launch_bounds__(256) k_eval_plain(ScanArgs a, int mol, long n,
     if (c.flags & REC_OUT_OF_GRID) atomicAdd((unsigned long long*)&a.counters[3], 1ull);
 }
 
+// The same with L lanes a point: each evaluates every L-th site into LDS, then
+// four of them add a component each in list order, so the sums are k_eval_plain's
+// to the bit (an absent Coulomb term adds +0 to a sum that is never -0).  Bound
+// by one point's chain: its terms (an LJ term is three divisions deep) and 16
+// cycles a site of ordered sum.  1000 points over 150 sites: 70 us with a lane a
+// point, 5 here.
+template <int L>
+__global__ void __launch_bounds__(256) k_eval_split(ScanArgs a, int mol, int n, const double* pos, double* out,
+                                                     int* off_grid) {
+    constexpr int PTS = 256 / L, ROW = L + 2, STRIDE = 8 * ROW + 2;   // + 2: values read together in different banks
+    __shared__ double lds[PTS * STRIDE];
+    const int lane = threadIdx.x % L, g = threadIdx.x / L;
+    const int p = blockIdx.x * PTS + g, pc = p < n ? p : n - 1;
+    const DevMol& m = a.mols[mol];
+    const Site64* sites = a.sites_ref + m.ref_off;
+    const V3 tip = {pos[3 * pc], pos[3 * pc + 1], pos[3 * pc + 2]};
+    double* mine = lds + g * STRIDE;
+    double acc = 0;
+    for (int im = 0; im < m.n_images; ++im) {
+        const double sx = m.shift[im][0], sy = m.shift[im][1], sz = m.shift[im][2];
+        for (int s0 = 0; s0 < m.n_sites; s0 += L) {
+            const int here = m.n_sites - s0 < L ? m.n_sites - s0 : L;
+            if (lane < here) {
+                const Site64 st = sites[s0 + lane];
+                const V3 r = {tip.x - (st.x + sx), tip.y - (st.y + sy), tip.z - (st.z + sz)};
+                const SiteTerms t = site_terms(st.vdw, st.coul, st.p0, st.p1, st.p2, st.qq, r);
+                double* o = mine + lane;
+                o[0] = t.f.x; o[ROW] = t.f.y; o[2 * ROW] = t.f.z; o[3 * ROW] = t.e;
+                o[4 * ROW] = t.fc.x; o[5 * ROW] = t.fc.y; o[6 * ROW] = t.fc.z; o[7 * ROW] = t.ec;
+            }
+            __syncthreads();
+            if (lane < 4) {
+                const double* o = mine + lane * ROW;
+                int k = 0;
+                for (; k + 8 <= here; k += 8) {
+                    double v[8], w[8];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) v[q] = o[k + q], w[q] = o[4 * ROW + k + q];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) {
+                        acc += v[q];
+                        acc += w[q];
+                    }
+                }
+                for (; k < here; ++k) {
+                    acc += o[k];
+                    acc += o[4 * ROW + k];
+                }
+            }
+            __syncthreads();
+        }
+    }
+    if (m.potential_grid >= 0) {
+        Ctx c = {&a, &m, 0};
+        V3 gf;
+        double ge;
+        grid_interp(c, a.grids[m.potential_grid], tip, gf, ge);
+        acc += lane == 0 ? gf.x : lane == 1 ? gf.y : lane == 2 ? gf.z : ge;
+        if (c.flags & REC_OUT_OF_GRID) *off_grid = 1;
+    }
+    if (lane < 4 && p < n) out[4 * p + lane] = acc;
+}
+
 // ForceGrid::interpolate (force_grid.cpp:88-155) of grid `grid` at
 // arbitrary positions; out-of-grid lookups counted in counters[3].
 __global__ void __launch_bounds__(256) k_grid_interp(ScanArgs a, int grid, long n, const double* pos, double* out) {
@@ -386,6 +447,18 @@ hipError_t launch_eval_plain(const ScanArgs& a, int mol, long n, const double* p
     int blocks = (int)((n + 255) / 256);
     if (blocks == 0) return hipSuccess;
     hipLaunchKernelGGL(k_eval_plain, dim3(blocks), dim3(256), 0, st, a, mol, n, pos, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_eval_split(const ScanArgs& a, int mol, int n, int lanes, const double* pos, double* out,
+                             int* off_grid, hipStream_t st) {
+    if (n <= 0) return hipSuccess;
+    const dim3 grid((unsigned)(((long)n * lanes + 255) / 256)), block(256);
+    switch (lanes) {
+        case 64: hipLaunchKernelGGL(k_eval_split<64>, grid, block, 0, st, a, mol, n, pos, out, off_grid); break;
+        case 16: hipLaunchKernelGGL(k_eval_split<16>, grid, block, 0, st, a, mol, n, pos, out, off_grid); break;
+        default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 
