@@ -1279,30 +1279,52 @@ static double flex_cost(int kind) {
 
 // The records of `terms` in the order the threads of a `waves`-wavefront block
 // evaluate them (FlexArgs::terms): the terms of each kind, in list order, are
-// cut into wave-rounds of 64, so the 64 lanes of a round run one code path, and
-// the rounds are dealt longest first, each to the wave with the least work so
-// far.  The last wave starts with `head` (it sums FIRE's power first).  Returns
-// the number of rounds.
+// cut into pieces of 64, so a wave runs one code path at a time, and the pieces
+// are dealt costliest first, each to the wave with the least work so far among
+// those that have room for it in the rounds whose terms stay in registers (a
+// round read from memory waits a microsecond for it); the ends of several kinds
+// share a round.  The last wave starts with `head` (it sums FIRE's power first).
+// Returns the number of rounds.
 static int flex_schedule(const std::vector<FxTerm>& terms, int waves, double head, std::vector<FxTerm>& out) {
     std::map<int, std::vector<int32_t>> by_kind;
     for (int k = 0; k < (int)terms.size(); ++k) by_kind[terms[k].kind].push_back(k);
-    struct Round {
+    struct Piece {
         double cost;
         const int32_t* terms;
         int n;
     };
-    std::vector<Round> rounds;
+    std::vector<Piece> pieces;
     for (const auto& kv : by_kind)
         for (size_t q = 0; q < kv.second.size(); q += 64)
-            rounds.push_back({flex_cost(kv.first), kv.second.data() + q, (int)std::min<size_t>(64, kv.second.size() - q)});
-    std::stable_sort(rounds.begin(), rounds.end(), [](const Round& x, const Round& y) { return x.cost > y.cost; });
+            pieces.push_back({flex_cost(kv.first), kv.second.data() + q, (int)std::min<size_t>(64, kv.second.size() - q)});
+    std::stable_sort(pieces.begin(), pieces.end(), [](const Piece& x, const Piece& y) { return x.cost > y.cost; });
+    struct Round {
+        int used = 0;
+        std::vector<const Piece*> pieces;
+    };
     std::vector<double> load(waves, 0.0);
     load[waves - 1] = head;
-    std::vector<std::vector<int>> mine(waves);
-    for (int r = 0; r < (int)rounds.size(); ++r) {
-        const int w = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-        load[w] += rounds[r].cost;
-        mine[w].push_back(r);
+    std::vector<std::vector<Round>> mine(waves);
+    auto room = [&](int w, int n) {   // the wave's round that takes n more terms; its next one
+        int r = 0;
+        while (r < (int)mine[w].size() && mine[w][r].used + n > 64) ++r;
+        return r;
+    };
+    for (const Piece& p : pieces) {
+        int best = -1;
+        bool best_held = false;
+        for (int w = 0; w < waves; ++w) {
+            const bool held = room(w, p.n) < FLEX_HELD_ROUNDS;
+            if (best < 0 || held > best_held || (held == best_held && load[w] < load[best])) {
+                best = w;
+                best_held = held;
+            }
+        }
+        const int r = room(best, p.n);
+        if (r == (int)mine[best].size()) mine[best].emplace_back();
+        mine[best][r].used += p.n;
+        mine[best][r].pieces.push_back(&p);
+        load[best] += p.cost;
     }
     int n_rounds = 0;
     for (const auto& m : mine) n_rounds = std::max(n_rounds, (int)m.size());
@@ -1313,48 +1335,53 @@ static int flex_schedule(const std::vector<FxTerm>& terms, int waves, double hea
     out.assign((size_t)n_rounds * T, none);
     for (int w = 0; w < waves; ++w)
         for (int r = 0; r < (int)mine[w].size(); ++r) {
-            const Round& R = rounds[mine[w][r]];
-            for (int l = 0; l < R.n; ++l) out[(size_t)r * T + 64 * w + l] = terms[R.terms[l]];
+            FxTerm* to = &out[(size_t)r * T + 64 * w];
+            for (const Piece* p : mine[w][r].pieces)
+                for (int l = 0; l < p->n; ++l) *to++ = terms[p->terms[l]];
         }
     return n_rounds;
 }
 
 // Device records of an interaction list: every term that acts on an atom whose
-// force is summed, its result slots (numbered per atom in the order
-// Interaction::eval adds to forces_[i]) and its places in the tip's energy list
-// (in the order it adds to energies_[1]).  idx: the kernels' index tables.
+// force is summed and its result slots (numbered per atom in the order
+// Interaction::eval adds to forces_[i], and for the tip to energies_[1]).
+// idx: the kernels' index tables.
 struct FlexList {
     std::vector<FxTerm> terms;
     std::vector<int32_t> idx;
-    int n_slots = 0, n_tip = 0, tip_rank = 0;
-    int tip_ts_slots = 0, tip_ts_terms = 0;   // of the first n_ts terms
+    int n_res = 0, n_tip = 0, n_rows = 0;
+    int tip_ts_slots = 0;   // of the first n_ts terms
 };
 
 static FlexList flex_list(int n, int n_terms, const mafm_flex_term* terms, int n_ts, const int32_t* fixed,
                           const std::vector<char>& summed) {
     FlexList L;
-    std::vector<int32_t> cnt(n, 0), order(n), rank(n);
+    std::vector<int32_t> cnt(n, 0), order, rank(n, 0);
     for (int k = 0; k < n_terms; ++k)
         for (int r = 0; r < flex_arity(terms[k].kind); ++r) cnt[terms[k].atom[r]] += summed[terms[k].atom[r]];
-    for (int i = 0; i < n; ++i) {
-        order[i] = i;
-        L.n_slots += cnt[i];
-    }
+    for (int i = 0; i < n; ++i)
+        if (i != 1) order.push_back(i);
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cnt[x] > cnt[y]; });
-    for (int k = 0; k < n; ++k) rank[order[k]] = k;
-    L.tip_rank = rank[1];
-    // row q: the q-th slots of the atoms that have more than q
-    std::vector<int32_t> row(cnt[order[0]] + 8, 0);
-    int width = n, at = 0;
-    for (int q = 0; q < cnt[order[0]]; ++q) {
-        while (width > 0 && cnt[order[width - 1]] <= q) --width;
-        row[q] = at;
-        at += 3 * width;
+    for (int k = 0; k < n - 1; ++k) rank[order[k]] = k;
+    L.n_tip = cnt[1];
+    const int others = 4 * flex_padded(L.n_tip);
+    // row q: slots 2 q and 2 q + 1 of the atoms that have more than 2 q
+    const int n_rows = (cnt[order[0]] + 1) / 2;
+    std::vector<int32_t> row((n_rows + 12 + 3) / 4 * 4, 0);
+    int width = n - 1;
+    L.n_res = others;
+    for (int q = 0; q < n_rows; ++q) {
+        while (width > 0 && cnt[order[width - 1]] <= 2 * q) --width;
+        row[q] = L.n_res - others;
+        L.n_res += 6 * width;
     }
-    for (int k = 0; k < n; ++k) L.idx.push_back(cnt[order[k]]);
+    L.n_rows = (int)row.size();
+    L.idx = row;
+    for (int k = 0; k < n - 1; ++k) L.idx.push_back(cnt[order[k]]);
+    L.idx.push_back(0);
     L.idx.insert(L.idx.end(), order.begin(), order.end());
+    L.idx.push_back(0);
     L.idx.insert(L.idx.end(), fixed, fixed + n);
-    L.idx.insert(L.idx.end(), row.begin(), row.end());
     std::vector<int32_t> next(n, 0);
     for (int k = 0; k < n_terms; ++k) {
         const mafm_flex_term& T = terms[k];
@@ -1364,9 +1391,9 @@ static FlexList flex_list(int n, int n_terms, const mafm_flex_term* terms, int n
         f.kind = T.kind;
         for (int r = 0; r < 4; ++r) {
             f.atom[r] = r < ar ? T.atom[r] : 0;
-            f.slot[r] = 3 * L.n_slots;
+            f.slot[r] = L.n_res;
         }
-        f.place[0] = f.place[1] = -1;
+        f.place[0] = f.place[1] = L.n_res;
         for (int q = 0; q < 6; ++q) f.q[q] = T.p[q];
         if (T.kind == MAFM_FX_LJ || T.kind == MAFM_FX_MORSE)
             for (int q = 0; q < 3; ++q) f.q[3 + q] = T.shift[q];
@@ -1376,21 +1403,17 @@ static FlexList flex_list(int n, int n_terms, const mafm_flex_term* terms, int n
             const int r = upd[q], i = T.atom[r];
             if (!summed[i]) continue;
             any = true;
-            f.slot[r] = row[next[i]++] + 3 * rank[i];
+            const int slot = next[i]++;
             if (i == 1) {
-                if (f.place[0] < 0) f.place[0] = L.n_tip++;
-                else f.place[1] = L.n_tip++;
-                if (k < n_ts) {
-                    ++L.tip_ts_slots;
-                    ++L.tip_ts_terms;
-                }
+                f.slot[r] = 8 * (slot / 2) + slot % 2;
+                f.place[f.place[0] == L.n_res ? 0 : 1] = f.slot[r] + 6;
+                if (k < n_ts) ++L.tip_ts_slots;
+            } else {
+                f.slot[r] = others + row[slot / 2] + 6 * rank[i] + slot % 2;
             }
         }
         if (any) L.terms.push_back(f);
     }
-    for (FxTerm& f : L.terms)
-        for (int q = 0; q < 2; ++q)
-            if (f.place[q] < 0) f.place[q] = L.n_tip;
     return L;
 }
 
@@ -1445,11 +1468,10 @@ mafm_status mafm_scan_flexible(mafm_ctx* c, const mafm_flex_desc* s, const mafm_
     FlexArgs a;
     memset(&a, 0, sizeof a);
     a.n_atoms = n;
-    a.n_slots = L.n_slots;
+    a.n_res = L.n_res;
     a.n_tip = L.n_tip;
     a.tip_ts_slots = L.tip_ts_slots;
-    a.tip_ts_terms = L.tip_ts_terms;
-    a.tip_rank = L.tip_rank;
+    a.n_rows = L.n_rows;
     a.nx = d->nx; a.ny = d->ny; a.nz = d->nz;
     a.dx = d->dx; a.dy = d->dy; a.dz = d->dz; a.zhigh = d->zhigh;
     a.minimiser = d->minimiser; a.integrator = d->integrator; a.minterm = d->minterm;
@@ -1471,7 +1493,7 @@ mafm_status mafm_scan_flexible(mafm_ctx* c, const mafm_flex_desc* s, const mafm_
     if (in_lds) per_cu = (int)std::max<size_t>(1, std::min<size_t>(per_cu, c->lds_per_cu / block_bytes));
     const int n_blocks = (int)std::min<long>(n_cols, (long)c->cus * per_cu);
     std::vector<FxTerm> sched;
-    a.rounds = flex_schedule(L.terms, waves, n / 20.0, sched);
+    a.rounds = flex_schedule(L.terms, waves, n / 10.0, sched);
 
     HIPCHK(c, c->d_fx_terms.reserve(std::max<size_t>(sched.size(), 1)));
     HIPCHK(c, c->d_fx_ints.reserve(ints.size()));
@@ -1568,7 +1590,8 @@ static mafm_status system_op(mafm_ctx* c, const mafm_interaction_list* L, int op
     SysArgs a;
     memset(&a, 0, sizeof a);
     a.n_atoms = n;
-    a.n_slots = list.n_slots;
+    a.n_res = list.n_res;
+    a.n_rows = list.n_rows;
     a.n_tip = list.n_tip;
     a.op = op;
     a.integrator = integrator;
@@ -1590,7 +1613,7 @@ static mafm_status system_op(mafm_ctx* c, const mafm_interaction_list* L, int op
     const int64_t blocks = std::min<int64_t>(n_states, 1 << 20);
     const size_t nd = sys_block_doubles(a);
     std::vector<FxTerm> sched;
-    a.rounds = flex_schedule(list.terms, waves, op == SYS_MINIMISE ? n / 20.0 : 0.0, sched);
+    a.rounds = flex_schedule(list.terms, waves, op == SYS_MINIMISE ? n / 10.0 : 0.0, sched);
 
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, c->d_fx_terms.reserve(std::max<size_t>(sched.size(), 1)));

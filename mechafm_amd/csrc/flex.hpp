@@ -6,17 +6,26 @@
 
 namespace mafm {
 
+constexpr int FLEX_HELD_ROUNDS = 4;   // rounds whose terms a thread keeps in registers
+
+// Lists that one thread sums (the atoms' powers, the tip's energies) are padded
+// to whole batches.
+constexpr int FLEX_BATCH = 16;
+__host__ __device__ inline int flex_padded(int n) { return (n + FLEX_BATCH - 1) / FLEX_BATCH * FLEX_BATCH; }
+
 // One interaction as the kernels read it.  Every term is evaluated once per
 // integrator stage into result slots {fx, fy, fz}, one per atom it acts on,
 // holding the signed force that atom receives (the reference's `forces[i] -= f`
 // is `+= -f`, the same rounding).  An atom's slots are numbered in the
-// interaction list's order, the order its force is summed in; slot q of the atom
-// of rank k (atoms by falling number of slots) has its components at row[q] + 3 k.
+// interaction list's order, the order its force is summed in.  They lie in pairs,
+// a slot's components two doubles apart: the tip's slot q, with its energy behind
+// the force, at 8 (q / 2) + q % 2; slot q of the other atom of rank k (by falling
+// number of slots) behind the tip's at row[q / 2] + 6 k + q % 2.
 struct FxTerm {
     int32_t kind;                     // MAFM_FX_*; -1: nothing to evaluate
     int32_t atom[4];
-    int32_t slot[4];                  // place of each atom's result slot; 3 n_slots: not read
-    int32_t place[2];                 // place of its energy in the tip's list; n_tip: not read
+    int32_t slot[4];                  // place of each atom's result slot; n_res: not read
+    int32_t place[2];                 // place of its energy where it acts on the tip; n_res: not read
     int32_t pad;
     double q[6];                      // pair terms: p0, p1, p2, shift x, y, z; else mafm_flex_term::p
 };
@@ -25,18 +34,19 @@ struct FxTerm {
 // r * block threads + l in rounds r < rounds.  The schedule only places the
 // work; the slots are summed in list order.
 struct FlexArgs {
-    int32_t n_atoms, n_slots, n_tip;  // n_tip: terms acting on the tip (an energy place each)
-    int32_t tip_ts_slots, tip_ts_terms;   // the tip's first slots / terms, from tip-surface terms
+    int32_t n_atoms, n_res, n_tip;    // doubles of results; slots of the tip
+    int32_t tip_ts_slots;             // the tip's first slots, from tip-surface terms
     int32_t nx, ny, nz;
     double dx, dy, dz, zhigh;
     int32_t minimiser, integrator, minterm, maxsteps;
     double etol, ftol, dt;
     const FxTerm* terms;
     int32_t rounds;
-    // index tables, back to back: slots of each rank (none for fixed atoms), its
-    // atom, fixed flags by atom (n_atoms each), the rows' places (and eight more)
+    // index tables, back to back: the rows' places (n_rows: 12 more than rows,
+    // rounded to whole fours), slots of each rank (none for fixed atoms; the last
+    // place is unused), its atom, fixed flags by atom (n_atoms each)
     const int32_t* idx;
-    int32_t tip_rank;
+    int32_t n_rows;
     const double* pos0;               // n_atoms x 3
     int32_t tip_pbc;
     int32_t state_col;                // column whose positions are kept per height, -1 none
@@ -54,7 +64,7 @@ struct FlexArgs {
 // minimisation from the given state.
 enum { SYS_EVAL = 0, SYS_STEP = 1, SYS_MINIMISE = 2 };
 struct SysArgs {
-    int32_t n_atoms, n_slots, n_tip, op;
+    int32_t n_atoms, n_res, n_tip, n_rows, op;
     int32_t minimiser, integrator, minterm, maxsteps;
     double etol, ftol, dt;
     int64_t n_states;

@@ -30,14 +30,16 @@
 // and square roots.  The angle, dihedral and Morse terms call the device acos /
 // sin / atan / exp, which may differ from glibc's in the last place.
 //
-// What bounds it: FP64 issue and the chain of one column -- a dihedral is three
-// roots, divisions and an atan deep.  The 72-atom graphene job at its full window
-// (12.8 M FIRE iterations, two columns a CU: their result slots fill the LDS):
-// 2285 vector instructions a wave and iteration, 45 % of the issue slots used
-// over the launch, the longest column 1.3 times the mean.  657 -> 473 ms, of
-// which terms in registers and component-parallel sums 657 -> 494, slots in rows
-// and shared divisions 494 -> 473; a relaxation of 300 states 20 -> 8.8 ms.
-// Bounded to 256 registers: at 268 one column a CU is resident, 712 ms.
+// What bounds it: one column's chain, FP64 operations that wait 8 cycles for the
+// one before, shared by two columns a CU (their result slots fill the LDS) whose
+// chains fill three quarters of the issue slots.  The 72-atom graphene job at its
+// full window (12.8 M FIRE iterations): an iteration 31000 -> 24800 cycles, of
+// which two evaluations take 16600 (an angle and a dihedral a lane each), force
+// sums and updates 5800, the mixing 1800; 657 -> 388 ms.  A relaxation of 300
+// states 19.7 -> 7.0 ms.  Measured on the way: an atom's slots side by side 494
+// ms, in rows of single values 473, pairs and the powers and the tip's sums as
+// padded lists 388; bounded to more than 256 registers (one column a CU) 712;
+// eight waves a column (one column a CU) 500.
 #include <algorithm>
 
 #include "flex.hpp"
@@ -65,7 +67,7 @@ __device__ inline V3 cross(V3 a, V3 b) {                                        
 }
 
 // A term as a thread holds it: the atoms it acts on, the result slot of each
-// (n_slots: nobody reads it), where the tip's energy list keeps its energy, and
+// (n_res: nobody reads it), where its energy goes if it acts on the tip, and
 // its numbers q (pair terms: p0, p1, p2, shift; the others: p).  Packed: 16-bit
 // pairs, for lists whose state fits the LDS.
 template <bool PACKED>
@@ -92,20 +94,28 @@ struct Term {
     }
 };
 
-// Where results go.  The slots lie in rows: row q holds the q-th slot of every
-// atom that has so many, the atoms by falling number of slots, three components
-// a slot, so the threads that sum one component each read neighbouring values
-// (an atom's slots side by side cost 6-way bank conflicts: 3300 against 900
-// cycles a sum phase).  A term's slot is its first component's place.
-//   E_TIP  energies of the tip's terms in their order, at tip[place]
-//   E_ALL  every atom's, at all[slot / 3]
+// Where results go: first the tip's slots, force and energy, which four lanes sum
+// side by side (the tip has a term with every surface atom, twice the slots of
+// the next); then the others' in rows: row q holds the slots 2 q and 2 q + 1 of
+// every atom that has so many, the atoms by falling number of slots, three
+// components a slot, so the threads that sum one component each read
+// neighbouring pairs (an atom's slots side by side cost 6-way bank conflicts;
+// values one by one, with their addresses, 46 instructions for eight against
+// 20).  A slot's components are two apart, its pair's other slot between; an
+// unpaired slot is paired with -0, which leaves every sum as it is.  A term's
+// slot is its first component's place; r[n_res] on takes what nobody reads.
+//   E_TIP  the tip's energies alone
+//   E_ALL  every atom's, the others' at all_place(slot)
 //   E_ONLY energies in a slot's first component, no forces
 enum { E_TIP = 0, E_ALL = 1, E_ONLY = 2 };
 struct Results {
     double* r;
-    double* tip;
     double* all;
-    int mode;
+    int others, n_res, mode;
+    __device__ int all_place(int slot) const {
+        const int q = (slot < others ? n_res : slot) - others;
+        return q / 6 * 2 + (q & 1);
+    }
 };
 
 template <bool P>
@@ -113,8 +123,8 @@ __device__ inline void put(const Results& R, const Term<P>& t, int role, V3 f) {
     double* r = R.r + t.slot(role);
     if (R.mode == E_ONLY) return;
     r[0] = f.x;
-    r[1] = f.y;
-    r[2] = f.z;
+    r[2] = f.y;
+    r[4] = f.z;
 }
 
 // One Interaction::eval of the list at positions X: the force on each atom
@@ -238,15 +248,14 @@ __device__ inline void eval_term(const Term<PACKED>& t, const double* X, const R
             break;
         }
     }
-    if (R.mode == E_TIP) {
-        R.tip[t.place(0)] = e_out;
-        R.tip[t.place(1)] = e_out;
-    } else {
-        for (int k = 0; k < roles; ++k) {
-            if (R.mode == E_ALL) R.all[t.slot(k) / 3] = e_out;
-            else R.r[t.slot(k)] = e_out;
-        }
+    if (R.mode == E_ONLY) {
+        for (int k = 0; k < roles; ++k) R.r[t.slot(k)] = e_out;
+        return;
     }
+    R.r[t.place(0)] = e_out;
+    R.r[t.place(1)] = e_out;
+    if (R.mode == E_ALL)
+        for (int k = 0; k < roles; ++k) R.all[R.all_place(t.slot(k))] = e_out;
 }
 
 // checkConvergence (minimiser.cpp:15-37)
@@ -261,77 +270,102 @@ __device__ inline bool converged(const A& a, V3 f, double ediff) {
 
 __device__ inline void block_sync() { __syncthreads(); }
 
-// acc + v[q0] + ... + v[q1 - 1], in order.  The additions are one chain; the
-// next eight values are in flight while eight are added.
-__device__ inline double seq_sum(double acc, const double* v, int q0, int q1) {
-    double r[8], s[8];
-    int q = q0;
-    if (q + 8 <= q1) {
+// A list that one thread sums is padded to whole batches with -0, and the batch
+// past its end may be read.
+constexpr int BATCH = FLEX_BATCH;
+
+// acc + the n values of a padded list, in order; its pairs are S apart.  One
+// chain of additions, the next batch in flight while one is added.  (By one lane
+// a masked or moved value costs as much as an addition: 95 cycles a value where
+// the batches were guarded.)
+template <int S>
+__device__ inline double list_sum(double acc, const double* v, int n) {
+    double2 r[BATCH / 2], s[BATCH / 2];
+    auto load = [&](double2* x, int q) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) r[j] = v[q + j];
-        for (; q + 16 <= q1; q += 8) {
+        for (int j = 0; j < BATCH / 2; ++j) x[j] = *reinterpret_cast<const double2*>(v + S * (q / 2 + j));
+    };
+    auto add = [&](const double2* x) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) s[j] = v[q + 8 + j];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) acc += r[j];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) r[j] = s[j];
+        for (int j = 0; j < BATCH / 2; ++j) {
+            acc += x[j].x;
+            acc += x[j].y;
         }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc += r[j];
-        q += 8;
-    }
-    // up to seven left: loaded together, added where they exist
-    const int left = q1 - q;
-    if (left > 0) {
-#pragma unroll
-        for (int j = 0; j < 7; ++j) s[j] = j < left ? v[q + j] : 0.0;
-#pragma unroll
-        for (int j = 0; j < 7; ++j)
-            if (j < left) acc += s[j];
+    };
+    load(r, 0);
+    for (int q = 0; q < n; q += 2 * BATCH) {
+        load(s, q + BATCH);
+        add(r);
+        if (q + BATCH >= n) break;
+        load(r, q + 2 * BATCH);
+        add(s);
     }
     return acc;
 }
 
-// acc + v[row[0] / div + p] + ... over the first nq rows, in order, as seq_sum.
-// The rows' places are read with scalar loads (the table has eight more).
+// acc + an atom's slots, in order: nq of them, pairs at v + row[0] / DIV + p,
+// v + row[1] / DIV + p, ...  Four pairs and the places of the four after them are
+// in flight while four are added; the table has twelve more rows, and past the
+// last one v is read but not added.
 template <int DIV>
-__device__ inline double row_sum(double acc, const double* v, cptr<int32_t> row, int nq, int p) {
-    double r[8], s[8];
-    int q = 0;
-    if (nq >= 8) {
+__device__ inline double row_sum(double acc, const double* v, const int32_t* row, int nq, int p) {
+    double2 r[4], s[4];
+    int4 w = *reinterpret_cast<const int4*>(row);
+    v += p;
+    auto load = [&](double2* x) {
+        x[0] = *reinterpret_cast<const double2*>(v + w.x / DIV);
+        x[1] = *reinterpret_cast<const double2*>(v + w.y / DIV);
+        x[2] = *reinterpret_cast<const double2*>(v + w.z / DIV);
+        x[3] = *reinterpret_cast<const double2*>(v + w.w / DIV);
+    };
+    auto places = [&](int q) { w = *reinterpret_cast<const int4*>(row + q); };
+    auto add = [&](const double2* x) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) r[j] = v[row[j] / DIV + p];
-        for (; q + 16 <= nq; q += 8) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) s[j] = v[row[q + 8 + j] / DIV + p];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) acc += r[j];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) r[j] = s[j];
+        for (int j = 0; j < 4; ++j) {
+            acc += x[j].x;
+            acc += x[j].y;
         }
+    };
+    const int n2 = (nq + 1) / 2;
+    load(r);
+    places(4);
+    int q = 0;
+    for (; q + 4 <= n2; q += 4) {
+        load(s);
+        places(q + 8);
+        add(r);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc += r[j];
-        q += 8;
+        for (int j = 0; j < 4; ++j) r[j] = s[j];
     }
-    const int left = nq - q;
-    if (left > 0) {
 #pragma unroll
-        for (int j = 0; j < 7; ++j) s[j] = j < left ? v[row[q + j] / DIV + p] : 0.0;
-#pragma unroll
-        for (int j = 0; j < 7; ++j)
-            if (j < left) acc += s[j];
+    for (int j = 0; j < 3; ++j) {
+        acc += q + j < n2 ? r[j].x : -0.0;
+        acc += q + j < n2 ? r[j].y : -0.0;
     }
     return acc;
 }
 
-// The force components a thread owns: places p = 3 rank + component, t, t +
-// block threads, ...; e = 3 atom + component, the entry in the state's arrays.
-#define FOR_ENTRIES(p, e) \
-    for (int p = t, e = entry_of(p); p < 3 * n; p += nthr, e = entry_of(p))
+// The force components a thread owns: of the other atoms the places p = 3 rank +
+// component, t, t + block threads, ...; the tip's go to the fourth to second
+// last thread, before its others (p past them all); the last thread has the tip's
+// energy.  e = 3 atom + component, the entry in the state's arrays.  What a
+// thread needs to know of its first place of the others stays in registers.
+struct Own {
+    int e, slots;
+    bool moves;
+};
+struct Places {
+    int t, nthr, n3, tip;    // tip: component of the tip, 3 its energy, < 0 neither
+    __device__ Places(int t_, int nthr_, int n) : t(t_), nthr(nthr_), n3(3 * (n - 1)), tip(t_ - (nthr_ - 4)) {}
+    __device__ int first() const { return (unsigned)tip < 3u ? n3 + tip : (t < n3 ? t : -1); }
+    __device__ int next(int p) const { return p >= n3 ? (t < n3 ? t : -1) : (p + nthr < n3 ? p + nthr : -1); }
+};
+#define FOR_ENTRIES(p, o)                                            \
+    for (int p = my.first(); p >= 0; p = my.next(p))                 \
+        if (const Own o = p >= my.n3 ? tip_own : p == t ? first : S.own(p); true)
 
 // Terms of a thread that stay in registers (lists whose state fits the LDS)
-constexpr int HELD_TERMS = 4;
+constexpr int HELD_TERMS = FLEX_HELD_ROUNDS;
 
 // The thread's terms of every round at positions X into R.
 template <bool PACKED>
@@ -364,35 +398,55 @@ struct Evaluator {
 };
 
 // Per-column state: positions, evaluation point, velocities, stage velocities
-// (then the mixed velocities), forces, powers, energies of the tip, broadcast
-// values, RK4's sums, results.
+// (then the mixed velocities), forces, powers, broadcast values, RK4's sums,
+// results.
 struct State {
-    double *pos, *pev, *vel, *vst, *frc, *pdot, *tip, *bc, *facc, *vacc, *eacc, *ener, *all, *res;
-    const int32_t *cnt, *order, *fixed;   // slots of each rank, its atom; fixed flags by atom
-    // the tables behind the state, copied from the rows' end on
-    __device__ void tables(const int32_t* idx, int n) {
-        cnt = idx;
-        order = idx + n;
-        fixed = idx + 2 * n;
+    double *pos, *pev, *vel, *vst, *frc, *pdot, *bc, *facc, *vacc, *eacc, *ener, *all, *res;
+    const int32_t *rows, *cnt, *order, *fixed;   // places of the rows; slots of each rank, its atom; fixed flags by atom
+    __device__ void tables(const int32_t* idx, int n_rows, int n) {
+        rows = idx;
+        cnt = rows + n_rows;
+        order = cnt + n;
+        fixed = order + n;
+    }
+    // the -0 that pad the lists and pair the unpaired slots (with_all: of the energies too)
+    __device__ void pad(int n, int n_tip, int others, bool with_all, int t, int nthr) {
+        for (int q = n + t; q < flex_padded(n); q += nthr) pdot[q] = -0.0;
+        for (int q = n_tip + t; q < flex_padded(n_tip); q += nthr)
+            for (int c = 0; c < 4; ++c) res[8 * (q / 2) + 2 * c + (q & 1)] = -0.0;
+        for (int k = t; k < n - 1; k += nthr) {
+            const int last = cnt[k] / 2;
+            if (cnt[k] % 2 == 0) continue;
+            for (int c = 0; c < 3; ++c) res[others + rows[last] + 6 * k + 2 * c + 1] = -0.0;
+            if (with_all) all[rows[last] / 3 + 2 * k + 1] = -0.0;
+        }
+    }
+    __device__ Own own(int p) const {
+        const int k = p / 3, i = order[k];
+        return {3 * i + (p - 3 * k), cnt[k], fixed[i] != 1};
     }
 };
-__host__ __device__ inline size_t flex_doubles(int n, int n_slots, int n_tip, bool rk4) {
-    return (size_t)(16 + (rk4 ? 6 : 0)) * n + (n_tip + 1) + 4 + 3 * ((size_t)n_slots + 1);
+// (the tables behind the state are read four at a time)
+__host__ __device__ inline size_t even(size_t doubles) { return doubles + (doubles & 1); }
+// What the sums may read past a list or a row of results is the state behind
+// them and, for the smallest systems, this.
+constexpr size_t SLACK = 8 * BATCH;
+__host__ __device__ inline size_t flex_doubles(int n, int n_res, bool rk4) {
+    return even(flex_padded(n) + 4 + n_res + 8 + (size_t)(15 + (rk4 ? 6 : 0)) * n);
 }
-__device__ inline State flex_layout(double* p, int n, int n_tip, bool rk4) {
+__device__ inline State flex_layout(double* p, int n, int n_res, bool rk4) {
     State S;
+    S.pdot = p; p += flex_padded(n);
+    S.bc = p; p += 4;
+    S.res = p; p += n_res + 8;
     S.pos = p; p += 3 * n;
     S.pev = p; p += 3 * n;
     S.vel = p; p += 3 * n;
     S.vst = p; p += 3 * n;
     S.frc = p; p += 3 * n;
-    S.pdot = p; p += n;
-    S.tip = p; p += n_tip + 1;
-    S.bc = p; p += 4;
     S.facc = p; p += rk4 ? 3 * n : 0;
-    S.vacc = p; p += rk4 ? 3 * n : 0;
+    S.vacc = p;
     S.eacc = S.ener = S.all = nullptr;
-    S.res = p;
     return S;
 }
 
@@ -409,31 +463,40 @@ __device__ inline double fire_mix(const State& S, int e, double alpha) {
 
 template <bool IN_LDS>
 __global__ void __launch_bounds__(256, 2) k_scan_flex(FlexArgs a) {
-    extern __shared__ double lds_flex[];
+    extern __shared__ __align__(16) double lds_flex[];
     __shared__ int col_shared;
     const int t = threadIdx.x;        // thread of the block (1-4 waves share a column)
     const int nthr = blockDim.x;
     const int n = a.n_atoms;
     const bool sd = a.minimiser == MAFM_MIN_SD, rk4 = !sd && a.integrator == MAFM_INT_RK4;
     const bool mid = !sd && a.integrator == MAFM_INT_MIDPOINT;
-    const size_t nd = flex_doubles(n, a.n_slots, a.n_tip, rk4);
-    double* base = IN_LDS ? lds_flex : a.work + (size_t)blockIdx.x * nd;
-    State S = flex_layout(base, n, a.n_tip, rk4);
+    const size_t nd = flex_doubles(n, a.n_res, rk4);
+    double* base = IN_LDS ? lds_flex : a.work + (size_t)blockIdx.x * (nd + SLACK);
+    State S = flex_layout(base, n, a.n_res, rk4);
     const int32_t* idx = a.idx;
     if (IN_LDS) {
         int32_t* l = reinterpret_cast<int32_t*>(lds_flex + nd);
-        for (int q = t; q < 3 * n; q += nthr) l[q] = a.idx[q];
+        for (int q = t; q < a.n_rows + 3 * n; q += nthr) l[q] = a.idx[q];
         idx = l;
     }
-    S.tables(idx, n);
-    const cptr<int32_t> rows = as_const(a.idx) + 3 * n;
-    const Results R = {S.res, S.tip, nullptr, E_TIP};
+    S.tables(idx, a.n_rows, n);
+    const int others = 4 * flex_padded(a.n_tip);
+    const Results R = {S.res, nullptr, others, a.n_res, E_TIP};
     Evaluator<IN_LDS> eval;
     eval.init(a.terms, a.rounds, t, nthr);
     block_sync();
-    auto entry_of = [&](int p) { return p < 3 * n ? 3 * S.order[p / 3] + p % 3 : 0; };
-    auto force = [&](int p) { return row_sum<1>(0.0, S.res, rows, S.cnt[p / 3], p); };
-    const int tip_place = 3 * a.tip_rank;
+    S.pad(n, a.n_tip, others, false, t, nthr);
+    const Places my(t, nthr, n);
+    const Own first = t < my.n3 ? S.own(t) : Own{0, 0, false};
+    const Own tip_own = {3 + my.tip, 0, true};
+    double tip_sum = 0;               // of the thread's component of the tip
+    auto sum_tip = [&]() {
+        if (my.tip >= 0) tip_sum = list_sum<8>(0.0, S.res + 2 * my.tip, a.n_tip);
+        if (my.tip == 3) S.bc[0] = tip_sum;   // read by the energy convergence test
+    };
+    auto force = [&](const Own& o, int p) {
+        return p >= my.n3 ? tip_sum : row_sum<1>(0.0, S.res + others, S.rows, o.slots, 2 * p);
+    };
     const int n_cols = a.nx * a.ny;
     for (;;) {
         if (t == 0) col_shared = atomicAdd(a.next_col, 1);
@@ -465,13 +528,13 @@ __global__ void __launch_bounds__(256, 2) k_scan_flex(FlexArgs a) {
         bool pending = false;         // mixed velocities wait in vst for P
         bool out = n_tot >= a.maxsteps;
         for (;;) {
-            if (pending && t == nthr - 1) S.bc[1] = seq_sum(0.0, S.pdot, 0, n);
+            if (pending && t == nthr - 1) S.bc[1] = list_sum<2>(0.0, S.pdot, n);
             eval(s == 0 || out ? S.pos : S.pev, R);
             block_sync();
             if (pending) {            // minimiser.cpp:107-126
                 const bool up = !(S.bc[1] < 0);
-                FOR_ENTRIES(p, e)
-                    if (S.fixed[e / 3] != 1) S.vel[e] = up ? S.vst[e] : 0.0;
+                FOR_ENTRIES(p, o)
+                    if (o.moves) S.vel[o.e] = up ? S.vst[o.e] : 0.0;
                 if (!up) {
                     nnn = 0;
                     dt *= 0.5;
@@ -490,8 +553,12 @@ __global__ void __launch_bounds__(256, 2) k_scan_flex(FlexArgs a) {
                 // getOutput (system.cpp:28-51): the tip-surface terms only
                 if (col == a.state_col && a.state)
                     for (int q = t; q < 3 * n; q += nthr) a.state[(size_t)k * 3 * n + q] = S.pos[q];
-                if (t < 3) S.frc[3 + t] = row_sum<1>(0.0, S.res, rows, a.tip_ts_slots, tip_place + t);
-                if (t == nthr - 1) S.bc[0] = seq_sum(0.0, S.tip, 0, a.tip_ts_terms);
+                if (my.tip >= 0) {
+                    double v = 0;
+#pragma unroll 8
+                    for (int q = 0; q < a.tip_ts_slots; ++q) v += S.res[8 * (q / 2) + 2 * my.tip + (q & 1)];
+                    *(my.tip == 3 ? S.bc : S.frc + 3 + my.tip) = v;
+                }
                 block_sync();
                 if (t == 0) {
                     const V3 d = ld3(S.pos, 0), r = ld3(S.pos, 1), f = ld3(S.frc, 1);
@@ -514,12 +581,12 @@ __global__ void __launch_bounds__(256, 2) k_scan_flex(FlexArgs a) {
                 out = n_tot >= a.maxsteps;
                 continue;
             }
-            // the tip's energy is read by the energy convergence test only
-            if (t == nthr - 1 && a.minterm != MAFM_TERM_F && !(mid && s == 0)) S.bc[0] = seq_sum(0.0, S.tip, 0, a.n_tip);
+            sum_tip();
             if (mid && s == 0) {            // midpointStep's half step
-                FOR_ENTRIES(p, e) {
-                    const double f = force(p), v = S.vel[e], x0 = S.pos[e];
-                    const bool free_ = S.fixed[e / 3] != 1;
+                FOR_ENTRIES(p, o) {
+                    const int e = o.e;
+                    const double f = force(o, p), v = S.vel[e], x0 = S.pos[e];
+                    const bool free_ = o.moves;
                     S.pev[e] = free_ ? x0 + dt / 2 * v : x0;
                     S.vst[e] = v + dt / 2 * f;
                 }
@@ -528,9 +595,10 @@ __global__ void __launch_bounds__(256, 2) k_scan_flex(FlexArgs a) {
                 continue;
             }
             if (rk4) {                                // stages at pos, pos + dt/2 v1, pos + dt/2 v2, pos + dt v3
-                FOR_ENTRIES(p, e) {
-                    const double fs = force(p), vs = s == 0 ? S.vel[e] : S.vst[e];
-                    const bool free_ = S.fixed[e / 3] != 1;
+                FOR_ENTRIES(p, o) {
+                    const int e = o.e;
+                    const double fs = force(o, p), vs = s == 0 ? S.vel[e] : S.vst[e];
+                    const bool free_ = o.moves;
                     double fa, va;
                     if (s == 0) { fa = fs; va = vs; }
                     else if (s < 3) { fa = S.facc[e] + 2 * fs; va = S.vacc[e] + 2 * vs; }
@@ -558,10 +626,11 @@ __global__ void __launch_bounds__(256, 2) k_scan_flex(FlexArgs a) {
                     continue;
                 }
             } else {
-                FOR_ENTRIES(p, e) {
-                    const double f = force(p);
+                FOR_ENTRIES(p, o) {
+                    const int e = o.e;
+                    const double f = force(o, p);
                     S.frc[e] = f;
-                    if (S.fixed[e / 3] != 1 && !sd) {  // midpointStep, eulerStep; masses are 1
+                    if (o.moves && !sd) {  // midpointStep, eulerStep; masses are 1
                         S.pos[e] = S.pos[e] + dt * (mid ? S.vst[e] : S.vel[e]);
                         S.vel[e] = S.vel[e] + dt * f;
                     }
@@ -577,10 +646,10 @@ __global__ void __launch_bounds__(256, 2) k_scan_flex(FlexArgs a) {
                 continue;
             }
             if (sd) {                                 // evaluate, test, move
-                FOR_ENTRIES(p, e)
-                    if (S.fixed[e / 3] != 1) S.pos[e] = S.pos[e] + a.dt * S.frc[e];
+                FOR_ENTRIES(p, o)
+                    if (o.moves) S.pos[o.e] = S.pos[o.e] + a.dt * S.frc[o.e];
             } else {
-                FOR_ENTRIES(p, e) S.vst[e] = fire_mix(S, e, alpha);
+                FOR_ENTRIES(p, o) S.vst[o.e] = fire_mix(S, o.e, alpha);
                 pending = true;
             }
             out = ++n_tot >= a.maxsteps;
@@ -597,57 +666,72 @@ __host__ __device__ inline bool sys_all_energies(const SysArgs& a) {
     return a.op != SYS_MINIMISE || (a.minimiser != MAFM_MIN_SD && a.integrator == MAFM_INT_RK4);
 }
 __host__ __device__ inline size_t sys_doubles(const SysArgs& a) {
-    return (size_t)24 * a.n_atoms + (a.n_tip + 1) + 4 + (sys_all_energies(a) ? 4 : 3) * ((size_t)a.n_slots + 1);
+    const size_t all = sys_all_energies(a) ? (a.n_res - 4 * flex_padded(a.n_tip)) / 3 + 2 : 0;
+    return even(flex_padded(a.n_atoms) + 4 + a.n_res + 8 + all + (size_t)23 * a.n_atoms);
 }
-__device__ inline State sys_layout(double* p, int n, int n_tip, int n_slots) {
+__device__ inline State sys_layout(double* p, const SysArgs& a) {
+    const int n = a.n_atoms;
     State S;
+    S.pdot = p; p += flex_padded(n);
+    S.bc = p; p += 4;
+    S.res = p; p += a.n_res + 8;
+    S.all = p; p += sys_all_energies(a) ? (a.n_res - 4 * flex_padded(a.n_tip)) / 3 + 2 : 0;
     S.pos = p; p += 3 * n;
     S.pev = p; p += 3 * n;
     S.vel = p; p += 3 * n;
     S.vst = p; p += 3 * n;
     S.frc = p; p += 3 * n;
-    S.pdot = p; p += n;
     S.facc = p; p += 3 * n;
     S.vacc = p; p += 3 * n;
     S.eacc = p; p += n;
-    S.ener = p; p += n;
-    S.tip = p; p += n_tip + 1;
-    S.bc = p; p += 4;
-    S.res = p; p += 3 * (n_slots + 1);
-    S.all = p;
+    S.ener = p;
     return S;
 }
 
 template <bool IN_LDS>
 __global__ void __launch_bounds__(256, 2) k_system_op(SysArgs a) {
-    extern __shared__ double lds_sys[];
+    extern __shared__ __align__(16) double lds_sys[];
     const int t = threadIdx.x, nthr = blockDim.x;
     const int n = a.n_atoms;
     const size_t nd = sys_doubles(a);
-    double* base = IN_LDS ? lds_sys : a.work + (size_t)blockIdx.x * nd;
-    State S = sys_layout(base, n, a.n_tip, a.n_slots);
+    double* base = IN_LDS ? lds_sys : a.work + (size_t)blockIdx.x * (nd + SLACK);
+    State S = sys_layout(base, a);
     const int32_t* idx = a.idx;
     if (IN_LDS) {
         int32_t* l = reinterpret_cast<int32_t*>(lds_sys + nd);
-        for (int q = t; q < 3 * n; q += nthr) l[q] = a.idx[q];
+        for (int q = t; q < a.n_rows + 3 * n; q += nthr) l[q] = a.idx[q];
         idx = l;
     }
-    S.tables(idx, n);
-    const cptr<int32_t> rows = as_const(a.idx) + 3 * n;
+    S.tables(idx, a.n_rows, n);
     const bool minimise = a.op == SYS_MINIMISE, sd = minimise && a.minimiser == MAFM_MIN_SD;
     const bool rk4 = !sd && a.op != SYS_EVAL && a.integrator == MAFM_INT_RK4;
     const bool mid = !sd && a.op != SYS_EVAL && a.integrator == MAFM_INT_MIDPOINT;
     const bool all_e = sys_all_energies(a);
-    Results R = {S.res, S.tip, S.all, all_e ? E_ALL : E_TIP};
+    const int others = 4 * flex_padded(a.n_tip);
+    Results R = {S.res, S.all, others, a.n_res, all_e ? E_ALL : E_TIP};
     Evaluator<IN_LDS> eval;
     eval.init(a.terms, a.rounds, t, nthr);
-    auto entry_of = [&](int p) { return p < 3 * n ? 3 * S.order[p / 3] + p % 3 : 0; };
-    auto force = [&](int p, double f0) { return row_sum<1>(f0, S.res, rows, S.cnt[p / 3], p); };
-    // every atom's energy from what `from` gives for it, into S.ener / S.eacc by `put`
+    block_sync();
+    S.pad(n, a.n_tip, others, all_e, t, nthr);
+    const Places my(t, nthr, n);
+    const Own first = t < my.n3 ? S.own(t) : Own{0, 0, false};
+    const Own tip_own = {3 + my.tip, 0, S.fixed[1] != 1};
+    double tip_sum = 0;               // of the thread's component of the tip, from f0 (its energy: e0)
+    auto sum_tip = [&](bool onto) {
+        if (my.tip < 0) return;
+        const double from = !onto ? 0.0 : my.tip == 3 ? S.ener[1] : S.frc[3 + my.tip];
+        tip_sum = list_sum<8>(from, S.res + 2 * my.tip, a.n_tip);
+        if (my.tip == 3) S.bc[0] = tip_sum;
+    };
+    auto force = [&](const Own& o, int p, double f0) {
+        return p >= my.n3 ? tip_sum : row_sum<1>(f0, S.res + others, S.rows, o.slots, 2 * p);
+    };
+    // every atom's energy into `to`, the others' from what `from` gives for them
     auto energies = [&](auto from, auto to) {
-        for (int k = t; k < n; k += nthr) {
+        if (my.tip == 3) to(1, tip_sum);
+        for (int k = t; k < n - 1; k += nthr) {
             const int i = S.order[k];
-            to(i, row_sum<3>(from(i), S.all, rows, S.cnt[k], k));
+            to(i, row_sum<3>(from(i), S.all, S.rows, S.cnt[k], 2 * k));
         }
     };
     block_sync();
@@ -671,9 +755,10 @@ __global__ void __launch_bounds__(256, 2) k_system_op(SysArgs a) {
         // minimiser.cpp:107-126, once P is there; P < 0 stops the fixed atoms too
         auto apply = [&]() {
             const bool up = !(S.bc[1] < 0);
-            FOR_ENTRIES(p, e) {
+            FOR_ENTRIES(p, o) {
+                const int e = o.e;
                 if (!up) S.vel[e] = 0;
-                else if (S.fixed[e / 3] != 1) S.vel[e] = S.vst[e];
+                else if (o.moves) S.vel[e] = S.vst[e];
             }
             if (!up) {
                 nnn = 0;
@@ -689,24 +774,28 @@ __global__ void __launch_bounds__(256, 2) k_system_op(SysArgs a) {
             pending = false;
         };
         while (run) {
-            if (pending && t == nthr - 1) S.bc[1] = seq_sum(0.0, S.pdot, 0, n);
+            if (pending && t == nthr - 1) S.bc[1] = list_sum<2>(0.0, S.pdot, n);
             R.mode = last ? E_ONLY : (all_e ? E_ALL : E_TIP);
             eval(s == 0 && !last ? S.pos : S.pev, R);
             block_sync();
             if (pending) apply();
             if (last) {
-                for (int k = t; k < n; k += nthr) S.ener[S.order[k]] = row_sum<1>(0.0, S.res, rows, S.cnt[k], 3 * k);
+                if (my.tip == 0) S.ener[1] = list_sum<8>(0.0, S.res, a.n_tip);
+                for (int k = t; k < n - 1; k += nthr)
+                    S.ener[S.order[k]] = row_sum<1>(0.0, S.res + others, S.rows, S.cnt[k], 6 * k);
                 break;
             }
+            sum_tip(onto);
             if (a.op == SYS_EVAL) {
-                FOR_ENTRIES(p, e) S.frc[e] = force(p, S.frc[e]);
+                FOR_ENTRIES(p, o) S.frc[o.e] = force(o, p, S.frc[o.e]);
                 energies([&](int i) { return S.ener[i]; }, [&](int i, double e) { S.ener[i] = e; });
                 break;
             }
             if (mid && s == 0) {                      // midpointStep's half step
-                FOR_ENTRIES(p, e) {
-                    const double f = force(p, 0.0), v = S.vel[e], x0 = S.pos[e];
-                    const bool free_ = S.fixed[e / 3] != 1;
+                FOR_ENTRIES(p, o) {
+                    const int e = o.e;
+                    const double f = force(o, p, 0.0), v = S.vel[e], x0 = S.pos[e];
+                    const bool free_ = o.moves;
                     S.pev[e] = free_ ? x0 + dt / 2 * v : x0;
                     S.vst[e] = free_ ? v + dt / 2 * f : v;
                 }
@@ -715,9 +804,10 @@ __global__ void __launch_bounds__(256, 2) k_system_op(SysArgs a) {
                 continue;
             }
             if (rk4) {                                // rk4Step
-                FOR_ENTRIES(p, e) {
-                    const double fs = force(p, 0.0), vs = s == 0 ? S.vel[e] : S.vst[e];
-                    const bool free_ = S.fixed[e / 3] != 1;
+                FOR_ENTRIES(p, o) {
+                    const int e = o.e;
+                    const double fs = force(o, p, 0.0), vs = s == 0 ? S.vel[e] : S.vst[e];
+                    const bool free_ = o.moves;
                     double fa, va;
                     if (s == 0) { fa = fs; va = vs; }
                     else if (s < 3) { fa = S.facc[e] + 2 * fs; va = S.vacc[e] + 2 * vs; }
@@ -747,10 +837,11 @@ __global__ void __launch_bounds__(256, 2) k_system_op(SysArgs a) {
                     continue;
                 }
             } else {
-                FOR_ENTRIES(p, e) {
-                    const double f = force(p, onto ? S.frc[e] : 0.0);
+                FOR_ENTRIES(p, o) {
+                    const int e = o.e;
+                    const double f = force(o, p, onto ? S.frc[e] : 0.0);
                     S.frc[e] = f;
-                    if (S.fixed[e / 3] != 1 && !sd) {
+                    if (o.moves && !sd) {
                         const double x0 = S.pos[e];
                         if (!mid) S.pev[e] = x0;      // where this step evaluated
                         S.pos[e] = x0 + dt * (mid ? S.vst[e] : S.vel[e]);
@@ -759,8 +850,6 @@ __global__ void __launch_bounds__(256, 2) k_system_op(SysArgs a) {
                 }
                 if (all_e) {
                     energies([&](int i) { return onto ? S.ener[i] : 0.0; }, [&](int i, double e) { S.ener[i] = e; });
-                } else if (t == nthr - 1 && a.minterm != MAFM_TERM_F) {
-                    S.bc[0] = seq_sum(0.0, S.tip, 0, a.n_tip);
                 }
                 block_sync();
             }
@@ -771,18 +860,18 @@ __global__ void __launch_bounds__(256, 2) k_system_op(SysArgs a) {
             const bool done = converged(a, ld3(S.frc, 1), e_tip - prev);
             if (!done) {
                 if (sd) {
-                    FOR_ENTRIES(p, e)
-                        if (S.fixed[e / 3] != 1) {
-                            S.pev[e] = S.pos[e];
-                            S.pos[e] = S.pos[e] + a.dt * S.frc[e];
+                    FOR_ENTRIES(p, o)
+                        if (o.moves) {
+                            S.pev[o.e] = S.pos[o.e];
+                            S.pos[o.e] = S.pos[o.e] + a.dt * S.frc[o.e];
                         }
                 } else {
-                    FOR_ENTRIES(p, e) S.vst[e] = fire_mix(S, e, alpha);
+                    FOR_ENTRIES(p, o) S.vst[o.e] = fire_mix(S, o.e, alpha);
                     pending = true;
                 }
                 ++n_tot;
             } else if (sd) {
-                FOR_ENTRIES(p, e) S.pev[e] = S.pos[e];
+                FOR_ENTRIES(p, o) S.pev[o.e] = S.pos[o.e];
             }
             block_sync();
             if (done || n_tot >= a.maxsteps) {
@@ -791,7 +880,7 @@ __global__ void __launch_bounds__(256, 2) k_system_op(SysArgs a) {
                     continue;
                 }
                 if (pending) {
-                    if (t == nthr - 1) S.bc[1] = seq_sum(0.0, S.pdot, 0, n);
+                    if (t == nthr - 1) S.bc[1] = list_sum<2>(0.0, S.pdot, n);
                     block_sync();
                     apply();
                 }
@@ -812,18 +901,20 @@ __global__ void __launch_bounds__(256, 2) k_system_op(SysArgs a) {
 
 }  // namespace
 
-size_t flex_block_doubles(const FlexArgs& a) {
-    return flex_doubles(a.n_atoms, a.n_slots, a.n_tip, a.minimiser == MAFM_MIN_FIRE && a.integrator == MAFM_INT_RK4);
+static size_t flex_state(const FlexArgs& a) {
+    return flex_doubles(a.n_atoms, a.n_res, a.minimiser == MAFM_MIN_FIRE && a.integrator == MAFM_INT_RK4);
 }
+
+size_t flex_block_doubles(const FlexArgs& a) { return flex_state(a) + SLACK; }
 
 size_t flex_block_lds(const FlexArgs& a) {
-    return flex_block_doubles(a) * sizeof(double) + 3 * (size_t)a.n_atoms * sizeof(int32_t);
+    return flex_state(a) * sizeof(double) + (a.n_rows + 3 * (size_t)a.n_atoms) * sizeof(int32_t);
 }
 
-size_t sys_block_doubles(const SysArgs& a) { return sys_doubles(a); }
+size_t sys_block_doubles(const SysArgs& a) { return sys_doubles(a) + SLACK; }
 
 size_t sys_block_bytes(const SysArgs& a) {
-    return sys_doubles(a) * sizeof(double) + 3 * (size_t)a.n_atoms * sizeof(int32_t);
+    return sys_doubles(a) * sizeof(double) + (a.n_rows + 3 * (size_t)a.n_atoms) * sizeof(int32_t);
 }
 
 hipError_t launch_system_op(const SysArgs& a, int waves, bool in_lds, hipStream_t st) {
