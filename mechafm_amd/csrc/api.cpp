@@ -451,6 +451,8 @@ static mafm_status build_tables(mafm_ctx* c, int n, const mafm_system_desc* sys,
             }
             d.n_seg[segk] = cnt;
         }
+        d.flat = 1;
+        for (int k = 1; k < s.n_sites; ++k) d.flat &= s.sites[k].z == s.sites[0].z;
         mols.push_back(d);
         cost.push_back(s.force_grid >= 0 ? 8 : std::max(1, s.n_sites * d.n_images));
     }
@@ -484,8 +486,9 @@ static bool product_images(const DevMol& d) {
 
 // Whether the whole-iteration kernels take these systems (FP64, Lennard-Jones
 // dummy), and in which mode: 0 Lennard-Jones (+ Coulomb) sites of one image
-// without an external potential, 1 force grids, 2 charge-free Lennard-Jones
-// sites with 3 x 3 product images, with or without a potential; -1 none.
+// without an external potential, 3 the same where each system's sites have one
+// height (flat molecules), 1 force grids, 2 charge-free Lennard-Jones sites with
+// 3 x 3 product images, with or without a potential; -1 none.
 static int iter_mode(const mafm_ctx* c, const std::vector<long>& cols, bool& coul) {
     int mode = -1;
     coul = false;
@@ -496,10 +499,13 @@ static int iter_mode(const mafm_ctx* c, const std::vector<long>& cols, bool& cou
         if (d.td_vdw != MAFM_VDW_LJ) return -1;
         if (d.force_grid >= 0) mine = 1;
         else if (d.n_seg[2] + d.n_seg[3] > 0) return -1;
-        else if (d.n_images == 1 && d.potential_grid < 0) mine = 0;
+        else if (d.n_images == 1 && d.potential_grid < 0) mine = d.flat ? 3 : 0;
         else if (product_images(d) && d.n_seg[0] == 0) mine = 2;
         else return -1;
-        if (mode >= 0 && mode != mine) return -1;
+        if (mode >= 0 && mode != mine) {
+            if (mode % 3 != 0 || mine % 3 != 0) return -1;
+            mine = 0;
+        }
         mode = mine;
         coul |= d.n_seg[0] > 0;
     }
@@ -510,16 +516,15 @@ static int iter_mode(const mafm_ctx* c, const std::vector<long>& cols, bool& cou
 // column (lanes = 0: chosen here).
 //
 // A wave's iteration costs about 45 instructions a site of a lane's share (260
-// with its nine images) plus
-// 330 (groups of up to 8 lanes) or 250 for the rest, so few lanes a column do
-// the least work, and many columns at once want few lanes.  Against that: a
-// wave alone on its SIMD issues an FP64 instruction every 8 cycles, two waves
-// together one every 4 (measured), so up to one wave a SIMD the time is that of
-// one wave; two waves a SIMD take 1.35 times as long; and columns past the
-// 2 waves a SIMD that fit wait for a second round, the last of which is
-// partly empty; and the more columns share a wave, the longer its last ones
-// run alone (4 % a factor of two).  The count with the least estimate is taken.  Measured, 96
-// charge-free sites, columns x lanes (ms): 2025 columns 64: 0.52, 32: 0.38,
+// with its nine images) plus 330 (groups of up to 8 lanes) or 250 for the rest,
+// so few lanes a column do the least work, and many columns at once want few
+// lanes.  Against that: an FP64 instruction that needs the last one's result
+// waits 8 cycles and issues in 4, so up to one wave a SIMD the time is that of
+// one wave and two waves a SIMD take 1.35 times as long; columns past the 2
+// waves a SIMD that fit wait for a second round, the last of which is partly
+// empty; and the more columns share a wave, the longer its last ones run alone
+// (4 % a factor of two).  The count with the least estimate is taken.  Measured,
+// 96 charge-free sites, columns x lanes (ms): 2025 columns 64: 0.52, 32: 0.38,
 // 16: 0.43; 10 201 columns 32: 1.87, 16: 1.38, 8: 1.77; 16 384 columns 16:
 // 2.13, 8: 1.89, 4: 2.37 (two lanes of the general kernel: 2.99, 5.0, 5.0).
 static void plan_iter(const mafm_ctx* c, const std::vector<long>& cols, int lanes, bool mid, FastPlan& p) {

@@ -14,16 +14,19 @@
 //   * groups of 16 and more lanes are summed on the FP64 matrix unit;
 //   * a force grid is read by eight lanes a column, one corner each, kept in
 //     registers until the cell changes.
-// What bounds it now: FP64 issue (a lone wave issues an FP64 instruction every
-// 8 cycles, two waves one every 4) and, for few columns, the length of the
-// longest column's chain.
+// What bounds it now: FP64 issue (4 cycles an instruction; one that needs the
+// last one's result waits 8, so two waves a SIMD fill the pipe) and, for few
+// columns, the length of the longest column's chain.
 // Measured (kernel ms, before -> now):
 //   one column over 96 sites                                      16.4 -> 3.2
-//   101 x 101 columns x 41 heights, 96 charge-free sites          26.5 -> 12.4
+//   101 x 101 columns x 41 heights, 96 charge-free flat sites     26.5 -> 12.5 (not as flat 13.2)
 //   33 x 33 x 41, RK4, 131 charged sites                          57 -> 16
 //   128 x 128 x 36 through a force grid                           26.4 -> 7.1
-//   128 x 128 x 30, 150 charged sites                             54.9 -> 23
-//   64 molecules of 20 to 400 charged sites, 64 x 64 x 40 each    406 -> 386
+//   128 x 128 x 30, 150 charged flat sites                        54.9 -> 18.6 (20.2)
+//   64 flat molecules of 20 to 400 charged sites, 64 x 64 x 40    406 -> 361 (392)
+// Tried and left out: flat or not decided in the kernel (RK4 17 -> 21: both
+// bodies' code and registers), charge-free sites sharing a reciprocal by fours
+// (the chain grows: one column 3.2 -> 3.9).
 //   64 x 64 x 40, 2000 sites with nine images and a potential     437 -> 244
 #include "../../include/mafm.h"
 #include <type_traits>
@@ -123,10 +126,12 @@ __device__ inline void group_sums(double* r) {
 // constants (q0 = 6 es6 / 2^8, q1 = 12 es12 / 2^14, qc = -qq / 2^3, all
 // exact), acc 3 collects 3 E.  Without Coulomb: q0 = 6 es6, q1 = 12 es12,
 // acc 3 collects 12 E.
-template <bool COUL, bool E>
-__device__ inline void pair_acc(const SiteLJ& st, double tx, double ty, double tz, double* acc) {
-    const double dx = tx - st.x, dy = ty - st.y, dz = tz - st.z;
-    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+// FLAT: the sites have one height, and tz is the tip's above it, dz2 its square;
+// acc 2 collects the force over tz (two instructions of 23 a charged site saved).
+template <bool COUL, bool E, bool FLAT>
+__device__ inline void pair_acc(const SiteLJ& st, double tx, double ty, double tz, double dz2, double* acc) {
+    const double dx = tx - st.x, dy = ty - st.y, dz = FLAT ? tz : tz - st.z;
+    const double r2 = fma(dx, dx, fma(dy, dy, FLAT ? dz2 : dz * dz));
     double fs;
     if (COUL) {
         const double z0 = __builtin_amdgcn_rsq(r2);
@@ -146,7 +151,7 @@ __device__ inline void pair_acc(const SiteLJ& st, double tx, double ty, double t
     }
     acc[0] = fma(fs, dx, acc[0]);
     acc[1] = fma(fs, dy, acc[1]);
-    acc[2] = fma(fs, dz, acc[2]);
+    acc[2] = FLAT ? acc[2] + fs : fma(fs, dz, acc[2]);
 }
 
 // One charge-free site and its 3 x 3 images: ax[i] / ay[j] = tip minus the
@@ -278,7 +283,8 @@ struct Grid {
 // What a column's tip-surface force is made of: the molecule's sites, a force
 // grid, or the sites' 3 x 3 periodic images and, where the system has one, an
 // external potential.
-enum { ITER_SITES = 0, ITER_GRID = 1, ITER_IMAGES = 2 };
+// ITER_FLAT: ITER_SITES where every molecule's sites have one height
+enum { ITER_SITES = 0, ITER_GRID = 1, ITER_IMAGES = 2, ITER_FLAT = 3 };
 
 // Sites of a lane that shares n sites with G - 1 others, padded: at least the
 // resident ones, and a multiple of two past them (res = 1, the images' kernels:
@@ -301,7 +307,7 @@ inline int resident_sites(int n, int G, bool mid) {
 // at a time.
 template <int G, int RES, bool COUL, int MODE, bool MID>
 __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanArgs& a) {
-    constexpr bool GRID = MODE == ITER_GRID, IMG = MODE == ITER_IMAGES;
+    constexpr bool GRID = MODE == ITER_GRID, IMG = MODE == ITER_IMAGES, FLAT = MODE == ITER_FLAT;
     const int lane = threadIdx.x & 63;
     const int gl = Lanes<G>::place(lane);
     const bool leader = gl == 0;
@@ -319,6 +325,7 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
     SiteLJ res[RES > 0 ? RES : 1];
     Dummy D;
     int per_lane = 0;                 // sites of a lane, a multiple of two past the resident ones
+    double flat_z = 0;                // their height where they have one
     // the corners last read, for the half steps and the full steps apart: a
     // pair of points on both sides of a cell face does not reload each other's
     Corner cn0 = {{0, 0, 0, 0}, -1}, cn1 = cn0;
@@ -359,6 +366,7 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
         }
         const int n = M->n_seg[0] + M->n_seg[1];
         per_lane = padded_share(n, G, RES);
+        if (FLAT) flat_z = n > 0 ? as_const(a.segf64)[M->seg_off].z + M->shift[0][2] : 0.0;
         __syncthreads();
         for (int t = threadIdx.x; t < per_lane * G; t += blockDim.x) {
             SiteLJ s = {1e4, 1e4, 1e4, 0, 0, 0};     // padding: no force, finite distance
@@ -489,8 +497,9 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
             if (E) r[3] *= 1.0 / 12.0;
         } else {
             r[0] = r[1] = r[2] = 0;
+            const double z = FLAT ? pz - flat_z : pz, dz2 = z * z;
 #pragma unroll
-            for (int u = 0; u < RES; ++u) pair_acc<COUL, E>(res[u], px, py, pz, r);
+            for (int u = 0; u < RES; ++u) pair_acc<COUL, E, FLAT>(res[u], px, py, z, dz2, r);
             if (per_lane > RES) {
                 // two sites in flight while two are evaluated, in turn
                 const SiteLJ* s = lsite + RES * G + gl;
@@ -501,19 +510,20 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
                         b0 = s[2 * G];
                         b1 = s[3 * G];
                     }
-                    pair_acc<COUL, E>(a0, px, py, pz, r);
-                    pair_acc<COUL, E>(a1, px, py, pz, r);
+                    pair_acc<COUL, E, FLAT>(a0, px, py, z, dz2, r);
+                    pair_acc<COUL, E, FLAT>(a1, px, py, z, dz2, r);
                     if (left <= 0) break;
                     s += 4 * G;
                     if (left > 2) {
                         a0 = s[0];
                         a1 = s[G];
                     }
-                    pair_acc<COUL, E>(b0, px, py, pz, r);
-                    pair_acc<COUL, E>(b1, px, py, pz, r);
+                    pair_acc<COUL, E, FLAT>(b0, px, py, z, dz2, r);
+                    pair_acc<COUL, E, FLAT>(b1, px, py, z, dz2, r);
                     if (left <= 2) break;
                 }
             }
+            if (FLAT) r[2] *= z;
             group_sums<G, E ? 4 : 3>(r);
             if (E) r[3] *= COUL ? 1.0 / 3.0 : 1.0 / 12.0;
         }
@@ -745,33 +755,33 @@ hipError_t launch_one(const IterLaunch& L) {
     return hipGetLastError();
 }
 
-template <int G, int RES, bool COUL, int MODE = ITER_SITES>
+template <int G, int RES, bool COUL, int MODE>
 hipError_t launch_mid(const IterLaunch& L) {
     return L.mid ? launch_one<G, RES, COUL, MODE, true>(L) : launch_one<G, RES, COUL, MODE, false>(L);
 }
 
-template <int G, bool COUL>
+template <int G, bool COUL, int MODE>
 hipError_t launch_res(const IterLaunch& L) {
     switch (resident_sites(L.n_min, G, L.mid)) {
-        case 2: return launch_mid<G, 2, COUL>(L);
-        case 3: return launch_mid<G, 3, COUL>(L);
-        case 4: return launch_mid<G, 4, COUL>(L);
-        case 5: return launch_mid<G, 5, COUL>(L);
-        case 6: return launch_mid<G, 6, COUL>(L);
+        case 2: return launch_mid<G, 2, COUL, MODE>(L);
+        case 3: return launch_mid<G, 3, COUL, MODE>(L);
+        case 4: return launch_mid<G, 4, COUL, MODE>(L);
+        case 5: return launch_mid<G, 5, COUL, MODE>(L);
+        case 6: return launch_mid<G, 6, COUL, MODE>(L);
         default:
-            if constexpr (G <= 8) return launch_one<G, 8, COUL, ITER_SITES, true>(L);
+            if constexpr (G <= 8) return launch_one<G, 8, COUL, MODE, true>(L);
             return hipErrorInvalidValue;
     }
 }
 
-template <bool COUL>
+template <bool COUL, int MODE>
 hipError_t launch_g(const IterLaunch& L, int G) {
     switch (G) {
-        case 4: return launch_res<4, COUL>(L);
-        case 8: return launch_res<8, COUL>(L);
-        case 16: return launch_res<16, COUL>(L);
-        case 32: return launch_res<32, COUL>(L);
-        case 64: return launch_res<64, COUL>(L);
+        case 4: return launch_res<4, COUL, MODE>(L);
+        case 8: return launch_res<8, COUL, MODE>(L);
+        case 16: return launch_res<16, COUL, MODE>(L);
+        case 32: return launch_res<32, COUL, MODE>(L);
+        case 64: return launch_res<64, COUL, MODE>(L);
         default: return hipErrorInvalidValue;
     }
 }
@@ -801,7 +811,8 @@ hipError_t launch_scan_iter(const ScanArgs& a, int G, bool coul, int mode, int n
             default: return hipErrorInvalidValue;
         }
     }
-    return coul ? launch_g<true>(L, G) : launch_g<false>(L, G);
+    if (mode == ITER_FLAT) return coul ? launch_g<true, ITER_FLAT>(L, G) : launch_g<false, ITER_FLAT>(L, G);
+    return coul ? launch_g<true, ITER_SITES>(L, G) : launch_g<false, ITER_SITES>(L, G);
 }
 
 }  // namespace mafm

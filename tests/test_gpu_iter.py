@@ -161,3 +161,26 @@ def test_periodic_images(gpu_ctx, n, potential):
         empty, keep2 = _system(0, False, rng)
         gpu_ctx.set_systems([empty])
         gpu_ctx.grid_free(h)
+
+
+@pytest.mark.parametrize("coul", [False, True])
+@pytest.mark.parametrize("n", [1, 5, 8, 16, 33, 64, 129, 260])
+def test_flat_molecules(gpu_ctx, n, coul):
+    """Sites of one height (their own kernels), off zero."""
+    d, keep = _system(n, coul, np.random.default_rng(100 + n))
+    for s in keep:
+        s.z = -0.37
+    _compare(gpu_ctx, [d], 5 * 3 * 6, lambda p, g: _desc(5, 3, 6, p, g))
+
+
+def test_flat_molecules_of_several_heights_and_one_buckled(gpu_ctx):
+    """A batch of flat molecules, each at its height, scans as flat; a buckled one among
+    them takes it to the general kernels."""
+    rng = np.random.default_rng(9)
+    made = [_system(n, True, rng) for n in (30, 12, 50)]
+    for k, (_, sites) in enumerate(made):
+        for s in sites:
+            s.z = 0.2 * k - 0.1
+    _compare(gpu_ctx, [d for d, _ in made], 3 * 4 * 3 * 5, lambda p, g: _desc(4, 3, 5, p, g))
+    made[1][1][3].z += 1e-3
+    _compare(gpu_ctx, [d for d, _ in made], 3 * 4 * 3 * 5, lambda p, g: _desc(4, 3, 5, p, g))
