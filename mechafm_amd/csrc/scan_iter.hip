@@ -24,10 +24,10 @@
 //   128 x 128 x 36 through a force grid                           26.4 -> 7.1
 //   128 x 128 x 30, 150 charged flat sites                        54.9 -> 18.6 (20.2)
 //   64 flat molecules of 20 to 400 charged sites, 64 x 64 x 40    406 -> 361 (392)
+//   64 x 64 x 40, 2000 sites with nine images and a potential     437 -> 244
 // Tried and left out: flat or not decided in the kernel (RK4 17 -> 21: both
 // bodies' code and registers), charge-free sites sharing a reciprocal by fours
 // (the chain grows: one column 3.2 -> 3.9).
-//   64 x 64 x 40, 2000 sites with nine images and a potential     437 -> 244
 #include "../../include/mafm.h"
 #include <type_traits>
 
@@ -91,8 +91,13 @@ struct Lanes {
 //   the group's sums either way: 0 x inf is NaN).  16 lanes, 3 values: 4 matrix
 //   instructions (16 cycles of the FP64 pipe each) and 6 moves against 36
 //   instructions of the butterflies.
+//   No addition here may be contracted with the product a caller's value comes
+//   from: a lane's a * b + (its neighbour's, rounded) is not its neighbour's sum,
+//   the lanes of a column then carry different states, and a long relaxation
+//   along a ridge drives them 1e-4 A apart.
 template <int G, int N>
 __device__ inline void group_sums(double* r) {
+#pragma clang fp contract(off)
     if constexpr (G <= 8) {
 #pragma unroll
         for (int q = 0; q < N; ++q) r[q] += dpp_f64<0xB1>(r[q]);

@@ -184,3 +184,21 @@ def test_flat_molecules_of_several_heights_and_one_buckled(gpu_ctx):
     _compare(gpu_ctx, [d for d, _ in made], 3 * 4 * 3 * 5, lambda p, g: _desc(4, 3, 5, p, g))
     made[1][1][3].z += 1e-3
     _compare(gpu_ctx, [d for d, _ in made], 3 * 4 * 3 * 5, lambda p, g: _desc(4, 3, 5, p, g))
+
+
+@pytest.mark.parametrize("lanes", [4, 8])
+def test_lanes_of_a_column_stay_together(gpu_ctx, tmp_path, lanes):
+    """Relaxations of thousands of iterations along a ridge, where one rounding
+    that differs between a column's lanes grows to 1e-4 A: a batch molecule at
+    its full window against the plain scan."""
+    from mechafm_amd import workloads as W
+    sim = abi.Simulation(W.make_c3(str(tmp_path))[18].input_path, gpu_ctx)
+    sim.run("plain64")
+    want = sim.records()
+    assert want["n_steps"].max() > 2000
+    sim.run("fast64", lanes_per_pixel=lanes)
+    got = sim.records()
+    np.testing.assert_array_equal(got["n_steps"], want["n_steps"])
+    for f in ("rx", "ry", "rz"):
+        assert np.abs(got[f] - want[f]).max() <= 1e-8
+    sim.close()
