@@ -116,6 +116,7 @@ struct ScanArgs {
     // sees the count.  Null: no counters.
     int32_t* col_done;
     int32_t lds_sites;        // scan_iter.hip: sites the LDS copy has room for
+    int32_t flat;             // scan_fast.hpp: every scanned molecule has sites of one height and one image
 };
 
 // Heights [0, heights) of column `gcol` are in host memory (ScanArgs::col_done).

@@ -124,6 +124,15 @@ struct Sites32 {
     }
 };
 
+// The flat layout of a staged site: A = {x, y, 6 es6 | 12 De, 12 es12 | a log2(e)},
+// B = {qq, a log2(e) re, 2 De a, z}.  A flat molecule's height is read once, so
+// an LJ pair takes one 16 B LDS read, LJ + Coulomb 16 + 4.
+__device__ inline void flat_site(float4& a, float4& b) {
+    const float z = a.z;
+    a = make_float4(a.x, a.y, a.w, b.x);
+    b = make_float4(b.y, b.z, b.w, z);
+}
+
 // Accumulators of the FP32 pair sums.
 //   ACC_BLOCK  FP32 partial sums over register blocks of sites, folded into FP64
 //   ACC_KAHAN  Kahan-compensated FP32 sum, term by term
@@ -171,9 +180,20 @@ struct Acc32 {
 
 // One site of segment SEG in registers: a = {x, y, z, 6 es6 | 12 De}, b = {12 es12 |
 // a log2(e), qq, - | a log2(e) re, - | 2 De a}; only the B words the segment uses
-// are read.
-template <int SEG, bool SC>
+// are read.  FLAT: from the flat layout of the LDS copy (flat_site).
+template <int SEG, bool SC, bool FLAT>
 __device__ inline void load_site(const Sites32<SC>& s, int t, float4& a, float4& b) {
+    if constexpr (FLAT) {
+        const float4 v = s.la[t];
+        a.x = v.x; a.y = v.y; a.w = v.z;
+        b.x = v.w;
+        if (SEG == 0) b.y = s.lb[t].x;
+        if (SEG >= 2) {
+            const float4 w = s.lb[t];
+            b.y = w.x; b.z = w.y; b.w = w.z;
+        }
+        return;
+    }
     a = s.A(t);
     if (SEG == 1) {
         b.x = s.B1(t);
@@ -256,18 +276,29 @@ __device__ inline void pair32(const float4 a, const float4 b, float tx, float ty
 // shifts are wave-uniform (scalar loads); the tip of image im is
 // t - shift[im] in FP32 relative to the molecule's origin.  IMG = false is
 // the single zero-shift image of a non-periodic system; E = false skips the
-// energy (the compiler drops its arithmetic).
-template <int SEG, bool SC, int MODE, bool IMG, bool E>
+// energy (the compiler drops its arithmetic).  FLAT (one image): every site of
+// the molecule has the height of the segment's first one, so dz and dz^2 are
+// formed once; the same values as site by site.
+template <int SEG, bool SC, int MODE, bool IMG, bool E, bool FLAT>
 __device__ inline void seg_sum32(cptr<DevMol> M, const Sites32<SC>& s, int n, int gl, int S, float tx, float ty,
                                  float tz, Acc32<MODE>& acc) {
     const int n_img = IMG ? M->n_images : 1;
     constexpr int B = SEG <= 1 ? 6 : 4;    // register blocks: 6 LJ sites (6 floats each), 4 Morse (8 floats)
     const int full = (n / (B * S)) * (B * S);
+    const float flat_dz = FLAT && n > 0 ? tz - s.lb[0].w : 0.f, flat_dz2 = flat_dz * flat_dz;
+    auto pair = [&](const float4& sa, const float4& sb, float ix, float iy, float iz) {
+        if constexpr (FLAT) {
+            const float dx = ix - sa.x, dy = iy - sa.y;
+            pair32_d<SEG, E>(sa, sb, dx, dy, flat_dz, fmaf(dx, dx, fmaf(dy, dy, flat_dz2)), acc);
+        } else {
+            pair32<SEG, E>(sa, sb, ix, iy, iz, acc);
+        }
+    };
     // one FP32 partial per register block (and all its images), folded into FP64
     for (int t0 = 0; t0 < full; t0 += B * S) {
         float4 sa[B], sb[B];
 #pragma unroll
-        for (int u = 0; u < B; ++u) load_site<SEG, SC>(s, t0 + u * S + gl, sa[u], sb[u]);
+        for (int u = 0; u < B; ++u) load_site<SEG, SC, FLAT>(s, t0 + u * S + gl, sa[u], sb[u]);
         acc.begin();
         if (IMG && M->planar) {
             // in-plane images: dz and dz^2 of a site are the same for all of them
@@ -295,7 +326,7 @@ __device__ inline void seg_sum32(cptr<DevMol> M, const Sites32<SC>& s, int n, in
                 }
 #pragma unroll
                 for (int u = 0; u < B; ++u) {
-                    pair32<SEG, E>(sa[u], sb[u], ix, iy, iz, acc);
+                    pair(sa[u], sb[u], ix, iy, iz);
                 }
             }
         }
@@ -304,7 +335,7 @@ __device__ inline void seg_sum32(cptr<DevMol> M, const Sites32<SC>& s, int n, in
     if (!IMG) acc.begin();
     for (int t = full + gl; t < n; t += S) {
         float4 sa, sb;
-        load_site<SEG, SC>(s, t, sa, sb);
+        load_site<SEG, SC, FLAT>(s, t, sa, sb);
         if (IMG) acc.begin();
         for (int im = 0; im < n_img; ++im) {
             float ix = tx, iy = ty, iz = tz;
@@ -313,35 +344,35 @@ __device__ inline void seg_sum32(cptr<DevMol> M, const Sites32<SC>& s, int n, in
                 iy -= M->shift32[im][1];
                 iz -= M->shift32[im][2];
             }
-            pair32<SEG, E>(sa, sb, ix, iy, iz, acc);
+            pair(sa, sb, ix, iy, iz);
         }
         if (IMG) acc.template end<E>();
     }
     if (!IMG) acc.template end<E>();
 }
 
-template <bool SC, int MODE, bool IMG, bool E>
+template <bool SC, int MODE, bool IMG, bool E, bool FLAT>
 __device__ inline void seg_sums32(cptr<DevMol> M, const Sites32<SC> s0, float tx, float ty, float tz, int gl, int S,
                                   Acc32<MODE>& acc) {
     Sites32<SC> s = s0;
     int n = M->n_seg[0];
-    seg_sum32<0, SC, MODE, IMG, E>(M, s, n, gl, S, tx, ty, tz, acc);
+    seg_sum32<0, SC, MODE, IMG, E, FLAT>(M, s, n, gl, S, tx, ty, tz, acc);
     s.advance(n);
     n = M->n_seg[1];
-    seg_sum32<1, SC, MODE, IMG, E>(M, s, n, gl, S, tx, ty, tz, acc);
+    seg_sum32<1, SC, MODE, IMG, E, FLAT>(M, s, n, gl, S, tx, ty, tz, acc);
     s.advance(n);
     n = M->n_seg[2];
-    if (n) seg_sum32<2, SC, MODE, IMG, E>(M, s, n, gl, S, tx, ty, tz, acc);
+    if (n) seg_sum32<2, SC, MODE, IMG, E, FLAT>(M, s, n, gl, S, tx, ty, tz, acc);
     s.advance(n);
     n = M->n_seg[3];
-    if (n) seg_sum32<3, SC, MODE, IMG, E>(M, s, n, gl, S, tx, ty, tz, acc);
+    if (n) seg_sum32<3, SC, MODE, IMG, E, FLAT>(M, s, n, gl, S, tx, ty, tz, acc);
 }
 
 // Sum of all tip-surface site terms of molecule M at tip position (px,py,pz):
 // this lane's share, sites gl, gl+S, ... of each segment (every image), S
 // lanes per position.  Coordinates are relative to the molecule's origin so
 // FP32 keeps ~1e-6 A resolution.
-template <bool SC, int MODE, bool E>
+template <bool SC, int MODE, bool E, bool FLAT>
 __device__ void site_sums32(cptr<DevMol> M, const Sites32<SC> s0, double px, double py, double pz, int gl, int S,
                             double out[4]) {
     Acc32<MODE> acc;
@@ -349,10 +380,10 @@ __device__ void site_sums32(cptr<DevMol> M, const Sites32<SC> s0, double px, dou
     const float tx = (float)(px - M->origin[0]);
     const float ty = (float)(py - M->origin[1]);
     const float tz = (float)(pz - M->origin[2]);
-    if (M->n_images > 1)
-        seg_sums32<SC, MODE, true, E>(M, s0, tx, ty, tz, gl, S, acc);
+    if (!FLAT && M->n_images > 1)
+        seg_sums32<SC, MODE, true, E, false>(M, s0, tx, ty, tz, gl, S, acc);
     else
-        seg_sums32<SC, MODE, false, E>(M, s0, tx, ty, tz, gl, S, acc);
+        seg_sums32<SC, MODE, false, E, FLAT>(M, s0, tx, ty, tz, gl, S, acc);
     out[0] = acc.get(0);
     out[1] = acc.get(1);
     out[2] = acc.get(2);
@@ -710,7 +741,7 @@ __device__ int next_rank(const ScanArgs& a, int rk) {
 // has finished its last column.
 // MID = true: FIRE with the midpoint integrator (the reference's default),
 // fixed at compile time so the RK4 / Euler / SD state is not allocated.
-template <int G, bool F32, int COMP, bool SC, bool MID>
+template <int G, bool F32, int COMP, bool SC, bool MID, bool FLAT = false>
 __device__ __attribute__((always_inline)) inline void scan_fast_body(const ScanArgs& a) {
     static_assert(!SC || G == 1, "scalar site streaming serves one lane per pixel");
     constexpr int B64 = MID ? 2 : 4;   // FP64 sites per register block
@@ -737,8 +768,10 @@ __device__ __attribute__((always_inline)) inline void scan_fast_body(const ScanA
             __syncthreads();
             if (F32) {
                 for (int t = threadIdx.x; t < n; t += blockDim.x) {
-                    lds_raw[t] = a.seg32a[Ms->seg_off + t];
-                    lds_raw[n + t] = a.seg32b[Ms->seg_off + t];
+                    float4 sa = a.seg32a[Ms->seg_off + t], sb = a.seg32b[Ms->seg_off + t];
+                    if (FLAT) flat_site(sa, sb);
+                    lds_raw[t] = sa;
+                    lds_raw[n + t] = sb;
                 }
             } else {
                 SiteF64* dst = reinterpret_cast<SiteF64*>(lds_raw);
@@ -872,8 +905,8 @@ __device__ __attribute__((always_inline)) inline void scan_fast_body(const ScanA
                         const float4* wa = SC ? a.seg32a + M->seg_off : lds_raw;
                         const float4* wb = SC ? a.seg32b + M->seg_off : lds_raw + lds_n;
                         Sites32<false> src64{wa, wb, wa, wb};
-                        if (need_e) site_sums32<false, COMP, true>(M, src64, qx, qy, qz, sub, Ge, part);
-                        else site_sums32<false, COMP, false>(M, src64, qx, qy, qz, sub, Ge, part);
+                        if (need_e) site_sums32<false, COMP, true, FLAT>(M, src64, qx, qy, qz, sub, Ge, part);
+                        else site_sums32<false, COMP, false, FLAT>(M, src64, qx, qy, qz, sub, Ge, part);
                     } else {
                         const SiteF64* w = SC ? a.segf64 + M->seg_off : reinterpret_cast<const SiteF64*>(lds_raw);
                         Sites<false, SiteF64> src64{w, w};
@@ -894,8 +927,8 @@ __device__ __attribute__((always_inline)) inline void scan_fast_body(const ScanA
             } else {
                 if constexpr (F32) {
                     Sites32<SC> src{a.seg32a + M->seg_off, a.seg32b + M->seg_off, lds_raw, lds_raw + lds_n};
-                    if (need_e) site_sums32<SC, COMP, true>(M, src, Px, Py, Pz, gl, G, r);
-                    else site_sums32<SC, COMP, false>(M, src, Px, Py, Pz, gl, G, r);
+                    if (need_e) site_sums32<SC, COMP, true, FLAT>(M, src, Px, Py, Pz, gl, G, r);
+                    else site_sums32<SC, COMP, false, FLAT>(M, src, Px, Py, Pz, gl, G, r);
                 } else {
                     Sites<SC, SiteF64> src{a.segf64 + M->seg_off, reinterpret_cast<const SiteF64*>(lds_raw)};
                     if (need_e) site_sums64<SC, true, B64>(M, src, Px, Py, Pz, gl, G, r);
@@ -1058,9 +1091,9 @@ __device__ __attribute__((always_inline)) inline void scan_fast_body(const ScanA
 // per SIMD (168 VGPRs; a few cold FIRE state values spill, which measured
 // faster than two waves without spills), the others to two waves (left free,
 // the compiler can take all 256 VGPRs and drop to one wave per SIMD).
-template <int G, int COMP, bool SC, bool MID>
+template <int G, int COMP, bool SC, bool MID, bool FLAT>
 __global__ void __launch_bounds__(512, MID ? 3 : 2) k_scan_fast32(ScanArgs a) {
-    scan_fast_body<G, true, COMP, SC, MID>(a);
+    scan_fast_body<G, true, COMP, SC, MID, FLAT>(a);
 }
 
 #ifndef MAFM_F64_MID_WAVES
@@ -1073,16 +1106,16 @@ __global__ void __launch_bounds__(512, MID ? MAFM_F64_MID_WAVES : 2) k_scan_fast
 
 // More than 64 KiB of dynamic LDS per workgroup (a molecule's sites staged
 // whole; gfx950 allows up to 160 KiB) has to be granted per kernel first.
-template <int G, bool F32, int COMP, bool MID, bool SC = false>
+template <int G, bool F32, int COMP, bool MID, bool SC = false, bool FLAT = false>
 hipError_t launch_one(const ScanArgs& a, int n_blocks, int W, size_t lds, hipStream_t st) {
     const size_t bytes = SC ? 0 : lds;
     if constexpr (F32) {
         if (bytes > 64 * 1024) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_scan_fast32<G, COMP, SC, MID>),
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_scan_fast32<G, COMP, SC, MID, FLAT>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
             if (e != hipSuccess) return e;
         }
-        hipLaunchKernelGGL((k_scan_fast32<G, COMP, SC, MID>), dim3(n_blocks), dim3(64 * W), bytes, st, a);
+        hipLaunchKernelGGL((k_scan_fast32<G, COMP, SC, MID, FLAT>), dim3(n_blocks), dim3(64 * W), bytes, st, a);
     } else {
         if (bytes > 64 * 1024) {
             const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_scan_fast64<G, SC, MID>),
@@ -1094,20 +1127,20 @@ hipError_t launch_one(const ScanArgs& a, int n_blocks, int W, size_t lds, hipStr
     return hipGetLastError();
 }
 
-template <bool F32, int COMP, bool MID>
+template <bool F32, int COMP, bool MID, bool FLAT = false>
 hipError_t launch_g(const ScanArgs& a, int G, bool scalar_sites, int n_blocks, int W, size_t lds, hipStream_t st) {
     if (scalar_sites) {
         if (G != 1) return hipErrorInvalidValue;
         return launch_one<1, F32, COMP, MID, true>(a, n_blocks, W, lds, st);
     }
     switch (G) {
-        case 1: return launch_one<1, F32, COMP, MID>(a, n_blocks, W, lds, st);
-        case 2: return launch_one<2, F32, COMP, MID>(a, n_blocks, W, lds, st);
-        case 4: return launch_one<4, F32, COMP, MID>(a, n_blocks, W, lds, st);
-        case 8: return launch_one<8, F32, COMP, MID>(a, n_blocks, W, lds, st);
-        case 16: return launch_one<16, F32, COMP, MID>(a, n_blocks, W, lds, st);
-        case 32: return launch_one<32, F32, COMP, MID>(a, n_blocks, W, lds, st);
-        case 64: return launch_one<64, F32, COMP, MID>(a, n_blocks, W, lds, st);
+        case 1: return launch_one<1, F32, COMP, MID, false, FLAT>(a, n_blocks, W, lds, st);
+        case 2: return launch_one<2, F32, COMP, MID, false, FLAT>(a, n_blocks, W, lds, st);
+        case 4: return launch_one<4, F32, COMP, MID, false, FLAT>(a, n_blocks, W, lds, st);
+        case 8: return launch_one<8, F32, COMP, MID, false, FLAT>(a, n_blocks, W, lds, st);
+        case 16: return launch_one<16, F32, COMP, MID, false, FLAT>(a, n_blocks, W, lds, st);
+        case 32: return launch_one<32, F32, COMP, MID, false, FLAT>(a, n_blocks, W, lds, st);
+        case 64: return launch_one<64, F32, COMP, MID, false, FLAT>(a, n_blocks, W, lds, st);
         default: return hipErrorInvalidValue;
     }
 }
@@ -1125,6 +1158,8 @@ hipError_t launch_scan_fast_family(const ScanArgs& a, bool f32, int comp, int G,
     const size_t lds = (size_t)lds_sites * 2 * sizeof(float4);
     if (comp == ACC_KAHAN) return launch_g<true, ACC_KAHAN, MID>(a, G, scalar_sites, n_blocks, W, lds, st);
     if (comp == ACC_NONE) return launch_g<true, ACC_NONE, MID>(a, G, scalar_sites, n_blocks, W, lds, st);
+    if constexpr (MID)
+        if (a.flat && !scalar_sites) return launch_g<true, ACC_BLOCK, MID, true>(a, G, false, n_blocks, W, lds, st);
     return launch_g<true, ACC_BLOCK, MID>(a, G, scalar_sites, n_blocks, W, lds, st);
 }
 
