@@ -533,8 +533,12 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
             if (E) r[3] *= COUL ? 1.0 / 3.0 : 1.0 / 12.0;
         }
     };
-    // the whole list: tip-surface plus, where with_d, tip-dummy
+    // the whole list: tip-surface plus, where with_d, tip-dummy.  The sum is never
+    // contracted with the product a dummy value comes from: it would be in the call
+    // whose with_d is known and not in the other, and a column's rounding would
+    // depend on whether a neighbour in its wave has a record to write.
     auto total = [&](auto want_e, Corner& cn, bool counts, bool with_d, double px, double py, double pz, double* r) {
+#pragma clang fp contract(off)
         constexpr bool E = decltype(want_e)::value;
         double d[4];
         dummy_terms<E>(D, dmx, dmy, dmz, px, py, pz, d);
