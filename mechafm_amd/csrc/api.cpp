@@ -610,7 +610,7 @@ static mafm_status plan_fast(mafm_ctx* c, const mafm_scan_desc* d, bool f32, con
         p.G = 1;
     }
     p.lds_sites = (int)max_sites;
-    a.flat = 1;
+    a.flat = 1;   // the FP32 kernels' rule; measured where they are launched
     for (int m = 0; m < n_mols; ++m)
         if (cols[m] > 0) a.flat &= c->mols[m].flat && c->mols[m].n_images == 1 && c->mols[m].force_grid < 0;
     // waves per workgroup share one LDS copy of the sites: grow W until the
