@@ -592,8 +592,11 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
         const double v2 = fma(vx, vx, fma(vy, vy, vz * vz));
         if (track) fire_margin(p, v2, v2 > 0 ? rsq64h(v2) : 0.0, mgp);
         // |v| / |f| by one root; 0 where the force has no direction (vectors.hpp:107-114)
-        const double vf = v2 * f2;
-        const double s = (f2 > 1e-20 && vf > 1e-280) ? alpha * v2 * rsq64h(vf) : 0.0;
+        // (beyond |f| = 2^200, where a tip was thrown off an atom, of the product over
+        // 2^1000: it would overflow where its factors do not)
+        const bool thrown = f2 > 0x1p400;
+        const double vf = v2 * (f2 * (thrown ? 0x1p-1000 : 1.0));
+        const double s = (f2 > 1e-20 && vf > 1e-280) ? alpha * (thrown ? 0x1p-500 : 1.0) * v2 * rsq64h(vf) : 0.0;
         const double b = 1 - alpha;
         const bool up = !(p < 0);
         vx = up ? fma(s, fx, b * vx) : 0.0;
