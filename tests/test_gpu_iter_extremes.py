@@ -58,3 +58,14 @@ def test_tip_thrown_off_an_atom(gpu_ctx, coul, flat):
     d, keep = _system([(0.0, 0.0, -1e-6), (0.0, 0.0, -1e-6 if flat else -2.0)], coul)
     want = _equal(gpu_ctx, d, 2, nz=2)
     assert np.isfinite(want["rz"]).all() and np.abs(want["rz"]).max() > 1e60
+
+
+@pytest.mark.parametrize("coul", [False, True])
+@pytest.mark.parametrize("flat", [False, True])
+@pytest.mark.parametrize("integrator", [0, 1, 2])
+def test_record_of_an_infinite_force(gpu_ctx, coul, flat, integrator):
+    """A record taken 1.7e-24 A from an atom: its force is infinite, its energy is not."""
+    a = 1e-24
+    d, keep = _system([(a, a, a), (1.0, 1.0, a if flat else -2.0)], coul)
+    want = _equal(gpu_ctx, d, 1, maxsteps=1, integrator=integrator)
+    assert np.isinf(want["fz"]).all() and np.isfinite(want["e"]).all()
