@@ -389,7 +389,9 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
         if (FLAT) flat_z = n > 0 ? as_const(a.segf64)[M->seg_off].z + M->shift[0][2] : 0.0;
         __syncthreads();
         for (int t = threadIdx.x; t < per_lane * G; t += blockDim.x) {
-            SiteLJ s = {1e4, 1e4, 1e4, 0, 0, 0};     // padding: no force, finite distance
+            // padding: no force, at a distance that is finite and never zero (nine
+            // images' squared distances are multiplied), where no scan goes
+            SiteLJ s = {1e15, 1e15, 1e15, 0, 0, 0};
             if (t < n) {
                 const SiteF64 f = a.segf64[M->seg_off + t];
                 s.x = f.x; s.y = f.y; s.z = f.z;

@@ -69,3 +69,17 @@ def test_record_of_an_infinite_force(gpu_ctx, coul, flat, integrator):
     d, keep = _system([(a, a, a), (1.0, 1.0, a if flat else -2.0)], coul)
     want = _equal(gpu_ctx, d, 1, maxsteps=1, integrator=integrator)
     assert np.isinf(want["fz"]).all() and np.isfinite(want["e"]).all()
+
+
+@pytest.mark.parametrize("coul", [False, True])
+@pytest.mark.parametrize("height", [0.0, 1e4])
+def test_scan_far_from_the_atoms(gpu_ctx, coul, height):
+    """A column 10 000 A off, its tip at 10 000 A in all three coordinates: the lanes'
+    padding is not there."""
+    d, keep = _system([(0.0, 0.0, height), (1.5, 0.0, height), (0.0, 1.5, height)], coul)
+    d.tip_dummy_d = 3.75
+    _equal(gpu_ctx, d, 4, nx=2, dx=1e4, zhigh=10003.75)
+    if not coul:
+        shifts = np.array([[i * 30.0, j * 30.0, 0.0] for i in (-1, 0, 1) for j in (-1, 0, 1)])
+        d.n_images, d.image_shifts = 9, shifts.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+        _equal(gpu_ctx, d, 4, lanes=(8, 16, 32, 64), nx=2, dx=1e4, zhigh=10003.75)
