@@ -78,15 +78,41 @@ struct SysArgs {
     int32_t* steps;    // n_states (minimise)
     double* work;      // per-block state when it does not fit LDS
 };
-size_t sys_block_doubles(const SysArgs& a);
-size_t sys_block_bytes(const SysArgs& a);   // with the index tables
 hipError_t launch_system_op(const SysArgs& a, int waves, bool in_lds, hipStream_t st);
 
-// Doubles of per-column state one block keeps (positions, integrator
-// stages, velocities, forces, term results).
-size_t flex_block_doubles(const FlexArgs& a);
+// Doubles of state a block keeps: the atoms' powers (a list), four broadcast
+// values, the results and eight more, then positions, integrator stages,
+// velocities and forces.  The sums load a batch past the end of a list and, of a
+// row, what wider rows have: both fall on the state behind the results, except
+// that with two or three atoms the tip's list needs more than there is.
+// Even: the index tables behind the state are read four at a time.
+__host__ __device__ inline size_t flex_state_doubles(int n, int n_res, int n_tip, size_t behind) {
+    const size_t own = n_res + 8 + behind, list = 4 * (size_t)(flex_padded(n_tip) + FLEX_BATCH);
+    const size_t all = flex_padded(n) + 4 + (own > list ? own : list);
+    return all + (all & 1);
+}
+__host__ __device__ inline size_t flex_block_doubles(const FlexArgs& a) {
+    const bool rk4 = a.minimiser == MAFM_MIN_FIRE && a.integrator == MAFM_INT_RK4;
+    return flex_state_doubles(a.n_atoms, a.n_res, a.n_tip, (size_t)(15 + (rk4 ? 6 : 0)) * a.n_atoms);
+}
 // LDS bytes of one block when the state lives there (state + index tables).
-size_t flex_block_lds(const FlexArgs& a);
+inline size_t flex_block_lds(const FlexArgs& a) {
+    return flex_block_doubles(a) * sizeof(double) + (a.n_rows + 3 * (size_t)a.n_atoms) * sizeof(int32_t);
+}
+
+// All energies of each evaluation are kept by eval, one step and RK4.
+__host__ __device__ inline bool sys_all_energies(const SysArgs& a) {
+    return a.op != SYS_MINIMISE || (a.minimiser != MAFM_MIN_SD && a.integrator == MAFM_INT_RK4);
+}
+__host__ __device__ inline size_t sys_energy_doubles(const SysArgs& a) {
+    return sys_all_energies(a) ? (a.n_res - 4 * flex_padded(a.n_tip)) / 3 + 2 : 0;
+}
+__host__ __device__ inline size_t sys_block_doubles(const SysArgs& a) {
+    return flex_state_doubles(a.n_atoms, a.n_res, a.n_tip, sys_energy_doubles(a) + (size_t)23 * a.n_atoms);
+}
+inline size_t sys_block_bytes(const SysArgs& a) {   // with the index tables
+    return sys_block_doubles(a) * sizeof(double) + (a.n_rows + 3 * (size_t)a.n_atoms) * sizeof(int32_t);
+}
 // waves: wavefronts per workgroup (1-4); in_lds: the state lives in LDS (else
 // in a.work, one slice per block).
 hipError_t launch_scan_flex(const FlexArgs& a, int n_blocks, int waves, bool in_lds, hipStream_t st);

@@ -426,14 +426,6 @@ struct State {
         return {3 * i + (p - 3 * k), cnt[k], fixed[i] != 1};
     }
 };
-// (the tables behind the state are read four at a time)
-__host__ __device__ inline size_t even(size_t doubles) { return doubles + (doubles & 1); }
-// What the sums may read past a list or a row of results is the state behind
-// them and, for the smallest systems, this.
-constexpr size_t SLACK = 8 * BATCH;
-__host__ __device__ inline size_t flex_doubles(int n, int n_res, bool rk4) {
-    return even(flex_padded(n) + 4 + n_res + 8 + (size_t)(15 + (rk4 ? 6 : 0)) * n);
-}
 __device__ inline State flex_layout(double* p, int n, int n_res, bool rk4) {
     State S;
     S.pdot = p; p += flex_padded(n);
@@ -470,8 +462,8 @@ __global__ void __launch_bounds__(256, 2) k_scan_flex(FlexArgs a) {
     const int n = a.n_atoms;
     const bool sd = a.minimiser == MAFM_MIN_SD, rk4 = !sd && a.integrator == MAFM_INT_RK4;
     const bool mid = !sd && a.integrator == MAFM_INT_MIDPOINT;
-    const size_t nd = flex_doubles(n, a.n_res, rk4);
-    double* base = IN_LDS ? lds_flex : a.work + (size_t)blockIdx.x * (nd + SLACK);
+    const size_t nd = flex_block_doubles(a);
+    double* base = IN_LDS ? lds_flex : a.work + (size_t)blockIdx.x * nd;
     State S = flex_layout(base, n, a.n_res, rk4);
     const int32_t* idx = a.idx;
     if (IN_LDS) {
@@ -661,21 +653,14 @@ __global__ void __launch_bounds__(256, 2) k_scan_flex(FlexArgs a) {
 // ---------------------------------------------------------------- System operators
 // State of one system copy: as the scan's, with every atom's energy, and a
 // fourth result component where the operator needs all energies of each
-// evaluation (eval, one step, RK4).
-__host__ __device__ inline bool sys_all_energies(const SysArgs& a) {
-    return a.op != SYS_MINIMISE || (a.minimiser != MAFM_MIN_SD && a.integrator == MAFM_INT_RK4);
-}
-__host__ __device__ inline size_t sys_doubles(const SysArgs& a) {
-    const size_t all = sys_all_energies(a) ? (a.n_res - 4 * flex_padded(a.n_tip)) / 3 + 2 : 0;
-    return even(flex_padded(a.n_atoms) + 4 + a.n_res + 8 + all + (size_t)23 * a.n_atoms);
-}
+// evaluation.
 __device__ inline State sys_layout(double* p, const SysArgs& a) {
     const int n = a.n_atoms;
     State S;
     S.pdot = p; p += flex_padded(n);
     S.bc = p; p += 4;
     S.res = p; p += a.n_res + 8;
-    S.all = p; p += sys_all_energies(a) ? (a.n_res - 4 * flex_padded(a.n_tip)) / 3 + 2 : 0;
+    S.all = p; p += sys_energy_doubles(a);
     S.pos = p; p += 3 * n;
     S.pev = p; p += 3 * n;
     S.vel = p; p += 3 * n;
@@ -693,8 +678,8 @@ __global__ void __launch_bounds__(256, 2) k_system_op(SysArgs a) {
     extern __shared__ __align__(16) double lds_sys[];
     const int t = threadIdx.x, nthr = blockDim.x;
     const int n = a.n_atoms;
-    const size_t nd = sys_doubles(a);
-    double* base = IN_LDS ? lds_sys : a.work + (size_t)blockIdx.x * (nd + SLACK);
+    const size_t nd = sys_block_doubles(a);
+    double* base = IN_LDS ? lds_sys : a.work + (size_t)blockIdx.x * nd;
     State S = sys_layout(base, a);
     const int32_t* idx = a.idx;
     if (IN_LDS) {
@@ -900,22 +885,6 @@ __global__ void __launch_bounds__(256, 2) k_system_op(SysArgs a) {
 }
 
 }  // namespace
-
-static size_t flex_state(const FlexArgs& a) {
-    return flex_doubles(a.n_atoms, a.n_res, a.minimiser == MAFM_MIN_FIRE && a.integrator == MAFM_INT_RK4);
-}
-
-size_t flex_block_doubles(const FlexArgs& a) { return flex_state(a) + SLACK; }
-
-size_t flex_block_lds(const FlexArgs& a) {
-    return flex_state(a) * sizeof(double) + (a.n_rows + 3 * (size_t)a.n_atoms) * sizeof(int32_t);
-}
-
-size_t sys_block_doubles(const SysArgs& a) { return sys_doubles(a) + SLACK; }
-
-size_t sys_block_bytes(const SysArgs& a) {
-    return sys_doubles(a) * sizeof(double) + (a.n_rows + 3 * (size_t)a.n_atoms) * sizeof(int32_t);
-}
 
 hipError_t launch_system_op(const SysArgs& a, int waves, bool in_lds, hipStream_t st) {
     const unsigned blocks = (unsigned)std::min<int64_t>(a.n_states, 1 << 20);
