@@ -307,6 +307,10 @@ mafm_status mafm_grid_upload(mafm_ctx* ctx, const mafm_grid_desc* grid, int* han
 mafm_status mafm_grid_build(mafm_ctx* ctx, const mafm_system_desc* sys, const mafm_grid_desc* grid,
                             int* handle);
 mafm_status mafm_grid_download(mafm_ctx* ctx, int handle, double* fe);
+/* The grid's memory (up to 512 MiB) stays with the context for the next grid of
+ * as many points, beside a workspace of up to 512 MiB.  Both go back to the device
+ * when an allocation of this context would fail without them, or when another
+ * grid is freed or a call needs a larger workspace, and with the context. */
 mafm_status mafm_grid_free(mafm_ctx* ctx, int handle);
 /* ForceGrid::interpolate (force_grid.hpp:33, force_grid.cpp:88-155) of grid
  * `handle` at n positions (n x 3): fe = n x 4 (fx fy fz e), the reference's

@@ -201,6 +201,7 @@ struct mafm_ctx {
     DevBuf<int64_t> d_counters;
     DevBuf<double> d_tmp;
     DevBuf<double> d_work;         // workspace of one call (transforms, adjoint, images): see Work
+    bool work_in_use = false;      // by the running call
     DevBuf<double4> spare64;       // the last freed grid's buffers, for the next grid
     DevBuf<float4> spare32;
     HostBuf<double> h_eval;        // points and results of a small tip-surface evaluation
@@ -254,19 +255,46 @@ static mafm_status fail(mafm_ctx* c, mafm_status s, const char* fmt, ...) {
 // Device memory a context keeps for the next call beyond its tables and
 // records: the workspace and one freed grid, each up to this size (hipFree waits
 // for the device and hipMalloc maps pages: 2 ms a potential of 2 M points).
+// An allocation of the context that fails takes them back.
 static constexpr size_t KEPT_BYTES = (size_t)512 << 20;
+
+// `allocate`, once more without the kept memory if the device has too little.
+template <typename F>
+static hipError_t with_kept_memory_back(mafm_ctx* c, F allocate) {
+    hipError_t e = allocate();
+    const bool work = c->d_work.p && !c->work_in_use;
+    if (e == hipErrorOutOfMemory && (c->spare64.p || c->spare32.p || work)) {
+        c->spare64.release();
+        c->spare32.release();
+        if (work) c->d_work.release();
+        e = allocate();
+    }
+    (void)hipGetLastError();   // a failed one is reported here, not by the next launch
+    return e;
+}
+
+template <typename T>
+static hipError_t device_alloc(mafm_ctx* c, T** p, size_t n) {
+    return with_kept_memory_back(c, [&] { return hipMalloc(p, n * sizeof(T)); });
+}
+
+template <typename T>
+static hipError_t grow(mafm_ctx* c, DevBuf<T>& b, size_t n) {
+    return with_kept_memory_back(c, [&] { return b.reserve(n); });
+}
 
 // The context's workspace for one call, which ends with the stream idle; a
 // large one is given back then.
 struct Work {
     mafm_ctx* c;
-    explicit Work(mafm_ctx* ctx) : c(ctx) {}
+    explicit Work(mafm_ctx* ctx) : c(ctx) { c->work_in_use = true; }
     Work(const Work&) = delete;
     Work& operator=(const Work&) = delete;
     ~Work() {
+        c->work_in_use = false;
         if (c->d_work.cap * sizeof(double) > KEPT_BYTES) c->d_work.release();
     }
-    hipError_t reserve(size_t doubles) { return c->d_work.reserve(doubles); }
+    hipError_t reserve(size_t doubles) { return grow(c, c->d_work, doubles); }
     double* p() const { return c->d_work.p; }
 };
 
@@ -285,7 +313,7 @@ static mafm_status sync_grids(mafm_ctx* c) {
         g.fe64 = h.fe64;
         g.fe32 = h.fe32;
     }
-    HIPCHK(c, c->d_grids.reserve(dg.size()));
+    HIPCHK(c, grow(c, c->d_grids, dg.size()));
     HIPCHK(c, hipMemcpyAsync(c->d_grids.p, dg.data(), dg.size() * sizeof(DevGrid), hipMemcpyHostToDevice,
                              c->stream));
     return MAFM_OK;
@@ -310,8 +338,8 @@ static mafm_status new_grid(mafm_ctx* c, const mafm_grid_desc* g, HostGrid& h) {
         h.fe64 = c->spare64.take();
         h.fe32 = c->spare32.take();
     } else {
-        HIPCHK(c, hipMalloc(&h.fe64, np * sizeof(double4)));
-        HIPCHK(c, hipMalloc(&h.fe32, np * sizeof(float4)));
+        HIPCHK(c, device_alloc(c, &h.fe64, np));
+        HIPCHK(c, device_alloc(c, &h.fe32, np));
     }
     h.live = true;
     return MAFM_OK;
@@ -700,9 +728,9 @@ static mafm_status plan_fast(mafm_ctx* c, const mafm_scan_desc* d, bool f32, con
         a.mol_order = dev_ws->order;
         return MAFM_OK;
     }
-    HIPCHK(c, c->d_next.reserve(n_mols));
-    HIPCHK(c, c->d_cum.reserve(n_mols + 1));
-    HIPCHK(c, c->d_order.reserve(n_mols));
+    HIPCHK(c, grow(c, c->d_next, n_mols));
+    HIPCHK(c, grow(c, c->d_cum, n_mols + 1));
+    HIPCHK(c, grow(c, c->d_order, n_mols));
     HIPCHK(c, hipMemcpyAsync(c->d_next.p, zero.data(), n_mols * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->d_cum.p, cum.data(), (n_mols + 1) * sizeof(float), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->d_order.p, order.data(), n_mols * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
@@ -846,7 +874,7 @@ mafm_status mafm_grid_interpolate(mafm_ctx* c, int handle, size_t n, const doubl
         return fail(c, MAFM_ERR_INVALID, "grid handle %d is not live", handle);
     if (n == 0) return MAFM_OK;
     HIPCHK(c, hipSetDevice(c->device));
-    HIPCHK(c, c->d_tmp.reserve(7 * n));
+    HIPCHK(c, grow(c, c->d_tmp, 7 * n));
     double* dpos = c->d_tmp.p;
     double* dout = c->d_tmp.p + 3 * n;
     HIPCHK(c, hipMemcpyAsync(dpos, pos, 3 * n * sizeof(double), hipMemcpyHostToDevice, c->stream));
@@ -869,7 +897,7 @@ mafm_status mafm_valu_calibration(mafm_ctx* c, int kind, int iterations, double*
     if (iterations < 1 || iterations > (1 << 20)) return fail(c, MAFM_ERR_INVALID, "iterations is %d", iterations);
     if (c->host_pending) return fail(c, MAFM_ERR_STATE, "a streamed scan is still running (mafm_scan_host_wait ends it)");
     HIPCHK(c, hipSetDevice(c->device));
-    HIPCHK(c, c->d_tmp.reserve(valu_calibration_doubles()));
+    HIPCHK(c, grow(c, c->d_tmp, valu_calibration_doubles()));
     int64_t insts = 0;
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     HIPCHK(c, launch_valu_calibration(kind, iterations, c->d_tmp.p, &insts, c->stream));
@@ -904,11 +932,11 @@ mafm_status mafm_grid_free(mafm_ctx* c, int handle) {
 
 static mafm_status upload_tables(mafm_ctx* c, const std::vector<DevMol>& mols, const std::vector<Site64>& ref,
                                  const std::vector<SiteF64>& seg64, const std::vector<Site32>& seg32) {
-    HIPCHK(c, c->d_mols.reserve(mols.size()));
-    HIPCHK(c, c->d_ref.reserve(ref.size()));
-    HIPCHK(c, c->d_seg64.reserve(seg64.size()));
-    HIPCHK(c, c->d_seg32a.reserve(seg32.size()));
-    HIPCHK(c, c->d_seg32b.reserve(seg32.size()));
+    HIPCHK(c, grow(c, c->d_mols, mols.size()));
+    HIPCHK(c, grow(c, c->d_ref, ref.size()));
+    HIPCHK(c, grow(c, c->d_seg64, seg64.size()));
+    HIPCHK(c, grow(c, c->d_seg32a, seg32.size()));
+    HIPCHK(c, grow(c, c->d_seg32b, seg32.size()));
     if (!mols.empty())
         HIPCHK(c, hipMemcpyAsync(c->d_mols.p, mols.data(), mols.size() * sizeof(DevMol), hipMemcpyHostToDevice, c->stream));
     if (!ref.empty())
@@ -1123,7 +1151,7 @@ static mafm_status scan_impl(mafm_ctx* c, const mafm_scan_desc* d, mafm_scan_sta
         c->have_scan = false;
         c->n_records = 0;
     } else {
-        HIPCHK(c, c->d_rec.reserve(n_rec));
+        HIPCHK(c, grow(c, c->d_rec, n_rec));
         c->n_records = n_rec;
         c->last_scan = *d;
         c->have_scan = true;
@@ -1142,7 +1170,7 @@ static mafm_status scan_impl(mafm_ctx* c, const mafm_scan_desc* d, mafm_scan_sta
     a.inv_2ftol = d->ftol > 0 ? 1.0 / (2.0 * d->ftol) : 0.0;
     const bool fast = d->precision != MAFM_PREC_PLAIN64;
     if (fast && (d->options & MAFM_SCAN_MARGINS)) {
-        HIPCHK(c, c->d_margins.reserve(n_rec));
+        HIPCHK(c, grow(c, c->d_margins, n_rec));
         a.margins = c->d_margins.p;
         c->have_margins = true;
     }
@@ -1503,13 +1531,13 @@ mafm_status mafm_scan_flexible(mafm_ctx* c, const mafm_flex_desc* s, const mafm_
     std::vector<FxTerm> sched;
     a.rounds = flex_schedule(L.terms, waves, n / 10.0, sched);
 
-    HIPCHK(c, c->d_fx_terms.reserve(std::max<size_t>(sched.size(), 1)));
-    HIPCHK(c, c->d_fx_ints.reserve(ints.size()));
-    HIPCHK(c, c->d_fx_pos.reserve(3 * (size_t)n));
-    HIPCHK(c, c->d_rec.reserve(n_rec));
-    HIPCHK(c, c->d_next.reserve(1));
-    if (s->state_column >= 0) HIPCHK(c, c->d_fx_state.reserve((size_t)d->nz * n * 3));
-    if (!in_lds) HIPCHK(c, c->d_fx_work.reserve((size_t)n_blocks * flex_block_doubles(a)));
+    HIPCHK(c, grow(c, c->d_fx_terms, std::max<size_t>(sched.size(), 1)));
+    HIPCHK(c, grow(c, c->d_fx_ints, ints.size()));
+    HIPCHK(c, grow(c, c->d_fx_pos, 3 * (size_t)n));
+    HIPCHK(c, grow(c, c->d_rec, n_rec));
+    HIPCHK(c, grow(c, c->d_next, 1));
+    if (s->state_column >= 0) HIPCHK(c, grow(c, c->d_fx_state, (size_t)d->nz * n * 3));
+    if (!in_lds) HIPCHK(c, grow(c, c->d_fx_work, (size_t)n_blocks * flex_block_doubles(a)));
     if (!sched.empty())
         HIPCHK(c, hipMemcpyAsync(c->d_fx_terms.p, sched.data(), sched.size() * sizeof(FxTerm), hipMemcpyHostToDevice,
                                  c->stream));
@@ -1624,10 +1652,10 @@ static mafm_status system_op(mafm_ctx* c, const mafm_interaction_list* L, int op
     a.rounds = flex_schedule(list.terms, waves, op == SYS_MINIMISE ? n / 10.0 : 0.0, sched);
 
     HIPCHK(c, hipSetDevice(c->device));
-    HIPCHK(c, c->d_fx_terms.reserve(std::max<size_t>(sched.size(), 1)));
-    HIPCHK(c, c->d_fx_ints.reserve(ints.size()));
-    HIPCHK(c, c->d_sys.reserve(3 * n3 + n1 + (n_states + 1) / 2 + 1));
-    if (!in_lds) HIPCHK(c, c->d_fx_work.reserve((size_t)blocks * nd));
+    HIPCHK(c, grow(c, c->d_fx_terms, std::max<size_t>(sched.size(), 1)));
+    HIPCHK(c, grow(c, c->d_fx_ints, ints.size()));
+    HIPCHK(c, grow(c, c->d_sys, 3 * n3 + n1 + (n_states + 1) / 2 + 1));
+    if (!in_lds) HIPCHK(c, grow(c, c->d_fx_work, (size_t)blocks * nd));
     double* d_pos = c->d_sys.p;
     double* d_vel = d_pos + n3;
     double* d_frc = d_vel + n3;
@@ -1783,7 +1811,7 @@ mafm_status mafm_eval_tip_surface(mafm_ctx* c, int system, size_t n, const doubl
         if (*off_grid) return fail(c, MAFM_ERR_OUT_OF_GRID, "tip position past the force grid");
         return MAFM_OK;
     }
-    HIPCHK(c, c->d_tmp.reserve(7 * n));
+    HIPCHK(c, grow(c, c->d_tmp, 7 * n));
     double* dpos = c->d_tmp.p;
     double* dout = c->d_tmp.p + 3 * n;
     HIPCHK(c, hipMemcpyAsync(dpos, pos, 3 * n * sizeof(double), hipMemcpyHostToDevice, c->stream));
@@ -1807,7 +1835,7 @@ static mafm_status twiddles_for(mafm_ctx* c, int n, const double2** out) {
         std::vector<double> h;
         fft_twiddles(n, h);
         DevBuf<double2>& b = c->twiddles[n];
-        hipError_t e = b.reserve(n);
+        hipError_t e = grow(c, b, n);
         if (e == hipSuccess)
             e = hipMemcpyAsync(b.p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
         if (e != hipSuccess) {
@@ -1891,7 +1919,7 @@ mafm_status mafm_potential_grid(mafm_ctx* c, const mafm_potential_desc* pd, int*
     double2* rho = pot + N;
     double2* tmp = rho + N;
     double* real = work.p() + 6 * N;
-    HIPCHK(c, c->d_flag.reserve(1));
+    HIPCHK(c, grow(c, c->d_flag, 1));
     HIPCHK(c, hipMemsetAsync(c->d_flag.p, 0, sizeof(int), c->stream));
     HIPCHK(c, hipMemcpyAsync(real, pd->potential, N * sizeof(double), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
@@ -1955,7 +1983,7 @@ mafm_status mafm_adjoint(mafm_ctx* c, int system, const mafm_adjoint_desc* d, ma
     double* g = dummy + 3 * n;
     double* v = g + n;
     double* out6 = v + 3 * n;
-    HIPCHK(c, c->d_flag.reserve(1));
+    HIPCHK(c, grow(c, c->d_flag, 1));
     HIPCHK(c, hipMemsetAsync(c->d_flag.p, 0, sizeof(int), c->stream));
     if (n) {
         HIPCHK(c, hipMemcpyAsync(tip, d->tip, 3 * n * sizeof(double), hipMemcpyHostToDevice, c->stream));
