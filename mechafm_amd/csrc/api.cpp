@@ -494,6 +494,7 @@ struct FastPlan {
     int G = 1, wps = 0, W = 1, n_blocks = 0, lds_sites = 0;
     bool scalar_sites = false, mid_family = false;
     bool iter = false, coul = false;                  // the whole-iteration kernels (scan_iter.hip)
+    bool one_lane = false;                            // the general kernels in their place, one lane a column
     int mode = -1;                                    // iter_mode
     int n_min = 0;                                    // fewest sites of a molecule with columns
 };
@@ -540,6 +541,53 @@ static int iter_mode(const mafm_ctx* c, const std::vector<long>& cols, bool& cou
     return mode;
 }
 
+// Whether the general kernels with one lane a column finish before the
+// whole-iteration ones, which take at least four lanes a column (eight for force
+// grids and images) and so keep four times the waves busy outside the site sums.
+// Once the columns fill the chip many times over that is all that counts; with
+// fewer the one lane's longer chain does.  rho is the ratio of the two times with
+// columns without end, and the line lies where the shrinking share of the chain
+// has let it through.  Measured, one lane over whole iterations, by columns:
+//   FIRE + midpoint, one molecule: 1 site 256^2 1.00, 400^2 0.71, 1000^2 0.55; 8 sites
+//     256^2 1.38, 400^2 1.00, 1000^2 0.80; 24 sites 640^2 1.15, 1000^2 0.98
+//   molecules of 64^2 columns (each one's last columns run in waves of few): 3 to 8
+//     sites, 16 molecules 1.09, 32: 0.67, 256: 0.43; 20 to 40 sites, 32: 1.30, 64:
+//     0.98, 256: 0.86; 20 to 100 sites, 128: 1.00
+//   RK4: 1 site 256^2 1.03, 1000^2 0.78; 8 sites 640^2 1.04.  SD and Euler: 4 sites 128^2
+//     1.85 and 1.70, 256^2 0.86 and 0.81; 80 sites 640^2 1.04 and 1.00
+//   force grid of 76 MB: 256^2 1.08, 320^2 0.93, 1000^2 0.68 (Euler 128^2 1.47, 200^2 0.81);
+//     of 487 MB, past the last-level cache: 320^2 1.17, 400^2 0.99, 720^2 0.86
+//   nine images: 2 sites 192^2 1.07, 256^2 0.68; 6 sites 256^2 1.34, 640^2 0.93; 16
+//     sites 640^2 1.33
+static bool one_lane_is_faster(const mafm_ctx* c, const mafm_scan_desc* d, const std::vector<long>& cols, int mode) {
+    const bool fire = d->minimiser == MAFM_MIN_FIRE, rk4 = fire && d->integrator == MAFM_INT_RK4;
+    const bool staged = rk4 || (fire && d->integrator == MAFM_INT_MIDPOINT);   // more than one evaluation an iteration
+    double total = 0, sites = 0, most = 0, grid_bytes = 0;
+    for (size_t m = 0; m < c->mols.size(); ++m) {
+        const DevMol& M = c->mols[m];
+        total += (double)cols[m];
+        sites += (double)cols[m] * M.n_sites;
+        most = std::max(most, (double)cols[m]);
+        if (mode != 1 || cols[m] <= 0) continue;
+        const HostGrid& g = c->grids[M.force_grid];
+        grid_bytes = std::max(grid_bytes, (double)g.n[0] * g.n[1] * g.n[2] * sizeof(double4));
+    }
+    if (total <= 0) return false;
+    const double n = sites / total;
+    if (mode == 1) return total >= (!staged ? 32e3 : grid_bytes > 256e6 ? 150e3 : 75e3);
+    if (mode == 2) {
+        const double rho = (staged ? 1.0 : 0.7) * (170 + 62 * n) / (260 * std::ceil(n / 8) + 330);
+        return total * (1 - rho) >= (staged ? 25e3 : 17e3);
+    }
+    const double drain = 100 * std::min(1.0, 4096 / most);
+    double rho = (190 + 16 * n) / (45 * std::ceil(n / 4) + 330 + drain);
+    if (rk4) rho += 0.15;
+    if (!staged) rho = 0.6 + n / (fire ? 400 : 200);
+    if (rho >= 1) return false;
+    const double from = (staged && !rk4 ? 40e3 : 20e3) * (std::pow(1 - rho, -1.4) - 1.4);
+    return total >= (most < 1024 ? from * std::max(1.0, n / 16) : from);
+}
+
 // Whether the whole-iteration kernels run this scan, and with how many lanes a
 // column (lanes = 0: chosen here).
 //
@@ -555,9 +603,15 @@ static int iter_mode(const mafm_ctx* c, const std::vector<long>& cols, bool& cou
 // 96 charge-free sites, columns x lanes (ms): 2025 columns 64: 0.52, 32: 0.38,
 // 16: 0.43; 10 201 columns 32: 1.87, 16: 1.38, 8: 1.77; 16 384 columns 16:
 // 2.13, 8: 1.89, 4: 2.37 (two lanes of the general kernel: 2.99, 5.0, 5.0).
-static void plan_iter(const mafm_ctx* c, const std::vector<long>& cols, int lanes, bool mid, FastPlan& p) {
+static void plan_iter(const mafm_ctx* c, const mafm_scan_desc* d, const std::vector<long>& cols, int lanes,
+                      FastPlan& p) {
+    const bool mid = d->minimiser == MAFM_MIN_FIRE && d->integrator == MAFM_INT_MIDPOINT;
     p.mode = iter_mode(c, cols, p.coul);
     if (p.mode < 0) return;
+    if (lanes == 0 && one_lane_is_faster(c, d, cols, p.mode)) {
+        p.one_lane = true;
+        return;
+    }
     int n_max = 1;
     long total = 0;
     p.n_min = INT32_MAX;
@@ -609,7 +663,7 @@ static mafm_status plan_fast(mafm_ctx* c, const mafm_scan_desc* d, bool f32, con
     p.mid_family = d->minimiser == MAFM_MIN_FIRE && d->integrator == MAFM_INT_MIDPOINT && !periodic;
     p.wps = waves_per_simd > 0 ? waves_per_simd : (p.mid_family ? 3 : 2);
     const bool mid = d->minimiser == MAFM_MIN_FIRE && d->integrator == MAFM_INT_MIDPOINT;
-    if (!f32) plan_iter(c, cols, lanes, mid, p);
+    if (!f32) plan_iter(c, d, cols, lanes, p);
     const long lanes_total = (long)c->cus * 4 * p.wps * 64;
     int64_t max_sites = 1;
     for (int m = 0; m < n_mols; ++m)
@@ -622,7 +676,7 @@ static mafm_status plan_fast(mafm_ctx* c, const mafm_scan_desc* d, bool f32, con
         p.G = 1;
         // split pixels over lanes until the columns give every resident lane
         // two pixels' share of work, and a lane keeps >= 8 sites
-        while (p.G < 64 && (double)total_cols * p.G < 2.0 * lanes_total && p.G * 8 <= max_sites) p.G <<= 1;
+        while (!p.one_lane && p.G < 64 && (double)total_cols * p.G < 2.0 * lanes_total && p.G * 8 <= max_sites) p.G <<= 1;
     }
     // a workgroup stages its molecule's sites in LDS (up to what one
     // workgroup may allocate, less 1 KiB for the kernel's static LDS: 159 KiB
