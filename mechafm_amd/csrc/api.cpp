@@ -493,7 +493,7 @@ static mafm_status build_tables(mafm_ctx* c, int n, const mafm_system_desc* sys,
 struct FastPlan {
     int G = 1, wps = 0, W = 1, n_blocks = 0, lds_sites = 0;
     bool scalar_sites = false, mid_family = false;
-    bool iter = false, coul = false;                  // the whole-iteration kernels (scan_iter.hip)
+    bool iter = false, coul = false;                  // the whole-iteration kernels (scan_iter.hpp)
     bool one_lane = false;                            // the general kernels in their place, one lane a column
     int mode = -1;                                    // iter_mode
     int n_min = 0;                                    // fewest sites of a molecule with columns

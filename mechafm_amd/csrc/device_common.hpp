@@ -115,7 +115,7 @@ struct ScanArgs {
     // so the host may read the column's first k + 1 records as soon as it
     // sees the count.  Null: no counters.
     int32_t* col_done;
-    int32_t lds_sites;        // scan_iter.hip: sites the LDS copy has room for
+    int32_t lds_sites;        // scan_iter.hpp: sites the LDS copy has room for
     int32_t flat;             // scan_fast.hpp: every scanned molecule has sites of one height and one image
 };
 

@@ -1,0 +1,9 @@
+// Whole-iteration scan kernels over sites of one height, the other minimisers and integrators.
+#include "scan_iter.hpp"
+
+namespace mafm {
+
+template hipError_t launch_iter_sites<false, ITER_FLAT, false>(const IterLaunch&, int);
+template hipError_t launch_iter_sites<true, ITER_FLAT, false>(const IterLaunch&, int);
+
+}  // namespace mafm

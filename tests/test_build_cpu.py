@@ -1,0 +1,30 @@
+"""How the library is built: what its kernels are bundled in, and what a changed
+header rebuilds."""
+import os
+import re
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "mechafm_amd", "csrc")
+LIB = os.path.join(ROOT, "mechafm_amd", "lib", "libmafm.so")
+
+
+@pytest.mark.skipif(not os.path.exists(LIB), reason="library not built")
+def test_kernels_are_loaded_in_small_parts():
+    """The runtime loads all kernels of a source file when the first one is
+    launched, 2 ms a MB, so a program's first scan pays for its whole file."""
+    data = open(LIB, "rb").read()
+    starts = [m.start() for m in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", data)]
+    assert len(starts) > 10
+    sizes = []
+    for s in starts:           # magic, number of entries, then offset, size and name length of each
+        at, total = s + 24, 0
+        n = int.from_bytes(data[at:at + 8], "little")
+        at += 8
+        for _ in range(n):
+            off, size, length = (int.from_bytes(data[at + 8 * k:at + 8 * k + 8], "little") for k in range(3))
+            total = max(total, off + size)
+            at += 24 + length
+        sizes.append(total)
+    assert max(sizes) <= 2.5e6, sorted(sizes)[-3:]
