@@ -22,6 +22,10 @@ class HostLink {
     // A transfer below this goes by one plain copy (1 MB: 0.07 ms plainly, 0.17
     // with threads to wake; 16 MB: 1.2 against 0.55).
     static constexpr size_t MIN_BYTES = 4u << 20;
+    // The ring and its threads take 0.7 to 1.4 ms to set up (5 in a process's first
+    // use), what they save on some 25 MB: a context that transfers less never has
+    // them (one 14 MB result of a fresh context: plainly 1.0 ms, with them 1.3).
+    static constexpr size_t OPEN_BYTES = 32u << 20;
 
     HostLink() = default;
     HostLink(const HostLink&) = delete;
@@ -30,7 +34,7 @@ class HostLink {
 
     // dst <- src (device memory) behind the work queued on st; complete on return.
     hipError_t to_host(void* dst, const void* src, size_t bytes, int device, hipStream_t st) {
-        if (bytes < MIN_BYTES || !pageable(dst) || !open(device)) {
+        if (bytes < MIN_BYTES || !pageable(dst) || !worth(bytes) || !open(device)) {
             hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
             return e == hipSuccess ? hipStreamSynchronize(st) : e;
         }
@@ -72,6 +76,7 @@ class HostLink {
     };
 
     char* ring_ = nullptr;
+    size_t plain_ = 0;                         // bytes of the transfers so far that it might have taken
     hipEvent_t ev_[SLOTS] = {};
     int n_ev_ = 0;
     bool failed_ = false;
@@ -91,6 +96,11 @@ class HostLink {
             return true;
         }
         return a.type == hipMemoryTypeUnregistered;
+    }
+
+    bool worth(size_t bytes) {
+        if (!ring_) plain_ += bytes;
+        return ring_ || plain_ >= OPEN_BYTES;
     }
 
     bool open(int device) {
