@@ -1852,7 +1852,9 @@ mafm_status mafm_eval_tip_surface(mafm_ctx* c, int system, size_t n, const doubl
     HIPCHK(c, hipSetDevice(c->device));
     const int lanes = eval_lanes(c->mols[system], n);
     if (lanes > 1 && n <= EVAL_MAPPED) {
-        HIPCHK(c, c->h_eval.reserve(7 * std::max<size_t>(n, 1024) + 1));
+        size_t room = 1024;   // by doubling: a caller whose points grow call by call allocates four times
+        while (room < n) room *= 2;
+        HIPCHK(c, c->h_eval.reserve(7 * room + 1));
         double* io = c->h_eval.p;
         double* dio = c->h_eval.dp;
         memcpy(io, pos, 3 * n * sizeof(double));
