@@ -1832,10 +1832,11 @@ mafm_status mafm_records(mafm_ctx* c, size_t first, size_t count, mafm_record* o
 // Lanes a point of the tip-surface operator: one lane a point leaves the chip
 // idle and walks the sites in series; more lanes pay for the ordered sum.  150
 // sites, us a call (1 / 16 / 64 lanes): one point 102 / 26 / 20, 1000 points 120 /
-// 28 / 24, 10000 points 146 / 92 / 96, 100000 points 463 / 464 / 535, 300000
-// points 1121 / 1192 / 1404.
+// 28 / 24, 10000 points 146 / 92 / 96.  The line (1 / 16 lanes): 8 sites, 30000
+// points 125 / 127, 60000 219 / 227; 150 sites, 90000 404 / 401, 110000 460 / 477,
+// 131072 513 / 547; 1000 sites, 90000 929 / 833, 110000 984 / 1006, 131072 1052 / 1174.
 static int eval_lanes(const DevMol& m, size_t n) {
-    if (m.force_grid >= 0 || n > 131072) return 1;
+    if (m.force_grid >= 0 || n > (m.n_sites < 64 ? 40000 : 90000)) return 1;
     return n <= 4096 && m.n_sites > 16 ? 64 : 16;
 }
 
