@@ -115,7 +115,19 @@ __device__ void eval_tip(Ctx& c, V3 dummy, V3 tip, bool ts_only, V3& F, double& 
             // positions[i2] + pbc_shift, subtracted from the tip (interactions.cpp:16)
             V3 r = {tip.x - (st.x + m.shift[im][0]), tip.y - (st.y + m.shift[im][1]),
                     tip.z - (st.z + m.shift[im][2])};
-            const SiteTerms t = site_terms(st.vdw, st.coul, st.p0, st.p1, st.p2, st.qq, r);
+            if (st.vdw == 0) {   // an LJ term shares nothing with its Coulomb term but r^2
+                V3 fv; double ev;
+                vdw(0, st.p0, st.p1, st.p2, r, fv, ev);
+                f.x += fv.x; f.y += fv.y; f.z += fv.z;
+                e += ev;
+                if (st.coul) {
+                    coulomb(st.qq, r, fv, ev);
+                    f.x += fv.x; f.y += fv.y; f.z += fv.z;
+                    e += ev;
+                }
+                continue;
+            }
+            const SiteTerms t = site_terms(1, st.coul, st.p0, st.p1, st.p2, st.qq, r);
             f.x += t.f.x; f.y += t.f.y; f.z += t.f.z;
             e += t.e;
             if (st.coul) {
