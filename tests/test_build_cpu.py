@@ -2,6 +2,7 @@
 header rebuilds."""
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -28,3 +29,33 @@ def test_kernels_are_loaded_in_small_parts():
             at += 24 + length
         sizes.append(total)
     assert max(sizes) <= 2.5e6, sorted(sizes)[-3:]
+
+
+def _includes(path, seen):
+    """Local headers a source includes, directly or through others."""
+    with open(path) as f:
+        for name in re.findall(r'^#include "([^"]+)"', f.read(), re.M):
+            p = os.path.normpath(os.path.join(os.path.dirname(path), name))
+            if p not in seen:
+                seen.add(p)
+                _includes(p, seen)
+    return seen
+
+
+def test_objects_depend_on_every_header_they_include():
+    """A changed header rebuilds each object that includes it (a stale one would be
+    tested and timed with the old code)."""
+    base = subprocess.run(["make", "-p", "-n", "all"], cwd=CSRC, capture_output=True, text=True, timeout=60).stdout
+    rules = {}
+    for m in re.finditer(r"^(\.\./lib/obj/\w+\.o):(?!=)(.*)$", base, re.M):
+        deps = [os.path.normpath(os.path.join(CSRC, d)) for d in m.group(2).replace("|", " ").split()]
+        rules.setdefault(os.path.basename(m.group(1)), set()).update(deps)
+    assert len(rules) > 12
+    missing = {}
+    for obj, deps in rules.items():
+        source = [d for d in deps if d.endswith((".hip", ".cpp"))]
+        assert len(source) == 1, (obj, source)
+        gone = _includes(source[0], set()) - deps
+        if gone:
+            missing[obj] = sorted(os.path.relpath(g, CSRC) for g in gone)
+    assert not missing, missing
