@@ -90,16 +90,16 @@ struct Lanes {
 //   the sums are then in lanes 0-3 of every quad and four DPP moves hand them
 //   out.  Products with 0 and 1 are exact, except that 0 x inf is NaN: one
 //   value's infinity makes the others NaN.  An iteration is lost either way (the
-//   mixing's |f| is infinite); RECORD, for the sums a record holds, adds such a
-//   group's values one by one.  16 lanes, 3 values: 4 matrix instructions (16
-//   cycles of the FP64 pipe each) and 6 moves against 36 instructions of the
-//   butterflies.
+//   mixing's |f| is infinite); for the sums a record holds (record) the values'
+//   row sums are picked by lane instead, the same bits where they are finite.  16
+//   lanes, 3 values: 4 matrix instructions (16 cycles of the FP64 pipe each) and 6
+//   moves against 36 instructions of the butterflies.
 //   No addition here may be contracted with the product a caller's value comes
 //   from: a lane's a * b + (its neighbour's, rounded) is not its neighbour's sum,
 //   the lanes of a column then carry different states, and a long relaxation
 //   along a ridge drives them 1e-4 A apart.
-template <int G, int N, bool RECORD>
-__device__ inline void group_sums(double* r) {
+template <int G, int N>
+__device__ inline void group_sums(double* r, bool record) {
 #pragma clang fp contract(off)
     if constexpr (G <= 8) {
 #pragma unroll
@@ -112,12 +112,19 @@ __device__ inline void group_sums(double* r) {
         }
     } else {
         const int lane = threadIdx.x & 63;
-        double d = 0.0, part[N];
+        double d = 0.0;
+        if (record) {
+            double row[N];
 #pragma unroll
-        for (int q = 0; q < N; ++q) part[q] = r[q];
+            for (int q = 0; q < N; ++q) row[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(r[q], 1.0, 0.0, 0, 0, 0);
+            d = row[0];
 #pragma unroll
-        for (int q = 0; q < N; ++q)
-            d = __builtin_amdgcn_mfma_f64_4x4x4f64(r[q], (lane & 3) == q ? 1.0 : 0.0, d, 0, 0, 0);
+            for (int q = 1; q < N; ++q) d = (lane & 3) == q ? row[q] : d;
+        } else {
+#pragma unroll
+            for (int q = 0; q < N; ++q)
+                d = __builtin_amdgcn_mfma_f64_4x4x4f64(r[q], (lane & 3) == q ? 1.0 : 0.0, d, 0, 0, 0);
+        }
         d = __builtin_amdgcn_mfma_f64_4x4x4f64(1.0, d, 0.0, 0, 0, 0);
         // blocks 0 + 1 and 2 + 3 (lane ^ 4 = half-row mirror of a mirrored quad),
         // then all four (lane ^ 8 = rotation by 8 within the row)
@@ -127,17 +134,6 @@ __device__ inline void group_sums(double* r) {
         r[1] = dpp_f64<0x55>(d);
         r[2] = dpp_f64<0xAA>(d);
         if (N > 3) r[3] = dpp_f64<0xFF>(d);
-        const bool finite = fabs(r[0]) < INFINITY;
-        if (RECORD && __any(!finite)) {
-#pragma unroll
-            for (int b = 1; b < 64; b <<= 1) {
-                if ((b == 4 && G < 32) || (b == 8 && G < 64)) continue;
-#pragma unroll
-                for (int q = 0; q < N; ++q) part[q] += __shfl_xor(part[q], b, 64);
-            }
-#pragma unroll
-            for (int q = 0; q < N; ++q) r[q] = finite ? r[q] : part[q];
-        }
     }
 }
 
@@ -477,8 +473,8 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
     };
     // tip-surface force and energy at p, summed over the group's lanes; record:
     // for some group's record
-    auto surface = [&](auto want_e, auto record, Corner& cn, bool counts, double px, double py, double pz, double* r) {
-        constexpr bool E = decltype(want_e)::value, REC = decltype(record)::value;
+    auto surface = [&](auto want_e, bool record, Corner& cn, bool counts, double px, double py, double pz, double* r) {
+        constexpr bool E = decltype(want_e)::value;
         r[3] = 0;
         if constexpr (GRID) {
             const double w = corner(cn, counts, px, py, pz);
@@ -486,7 +482,7 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
             r[1] = w * cn.v.y;
             r[2] = w * cn.v.z;
             if (E) r[3] = w * cn.v.w;
-            group_sums<G, E ? 4 : 3, REC>(r);
+            group_sums<G, E ? 4 : 3>(r, record);
         } else if constexpr (IMG) {
             r[0] = r[1] = r[2] = 0;
             if (has_grid && gl < 8) {   // eight of the column's lanes hold the potential's corners
@@ -517,7 +513,7 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
                 q1 = q2;
             }
             images_acc<E>(st, q1, ax, ay, pz, r);
-            group_sums<G, E ? 4 : 3, REC>(r);
+            group_sums<G, E ? 4 : 3>(r, record);
             if (E) r[3] *= 1.0 / 12.0;
         } else {
             r[0] = r[1] = r[2] = 0;
@@ -548,7 +544,7 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
                 }
             }
             if (FLAT) r[2] *= z;
-            group_sums<G, E ? 4 : 3, REC>(r);
+            group_sums<G, E ? 4 : 3>(r, record);
             if (E) r[3] *= COUL ? 1.0 / 3.0 : 1.0 / 12.0;
         }
     };
@@ -556,7 +552,7 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
     // contracted with the product a dummy value comes from: it would be in the call
     // whose with_d is known and not in the other, and a column's rounding would
     // depend on whether a neighbour in its wave has a record to write.
-    auto total = [&](auto want_e, auto record, Corner& cn, bool counts, bool with_d, double px, double py, double pz,
+    auto total = [&](auto want_e, bool record, Corner& cn, bool counts, bool with_d, double px, double py, double pz,
                      double* r) {
 #pragma clang fp contract(off)
         constexpr bool E = decltype(want_e)::value;
@@ -566,8 +562,6 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
 #pragma unroll
         for (int q = 0; q < (E ? 4 : 3); ++q) r[q] += with_d ? d[q] : 0.0;
     };
-    constexpr std::true_type yes{};
-    constexpr std::false_type no{};
     auto begin_height = [&]() {
         n_tot = 1; dt = a.dt; alpha = 0.1; nnn = 0; flags = 0;
         mgf = mge = mgp = INFINITY;
@@ -694,13 +688,13 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
             // finished height at theirs (tip-surface terms only)
             const double hx = dt / 2 * vx, hy = dt / 2 * vy, hz = dt / 2 * vz;
             if (__any(emits)) {
-                total(yes, yes, cn0, true, !emits, tx, ty, tz, r);
+                total(std::true_type{}, true, cn0, true, !emits, tx, ty, tz, r);
                 if (emits) emit(r);
             } else {
-                total(no, no, cn0, true, true, tx, ty, tz, r);
+                total(std::false_type{}, false, cn0, true, true, tx, ty, tz, r);
             }
             const double ax = fma(dt / 2, r[0], vx), ay = fma(dt / 2, r[1], vy), az = fma(dt / 2, r[2], vz);
-            total(yes, no, cn1, live, true, tx + hx, ty + hy, tz + hz, r);
+            total(std::true_type{}, false, cn1, live, true, tx + hx, ty + hy, tz + hz, r);
             if (live) {
                 tx = fma(dt, ax, tx); ty = fma(dt, ay, ty); tz = fma(dt, az, tz);
                 vx = fma(dt, r[0], vx); vy = fma(dt, r[1], vy); vz = fma(dt, r[2], vz);
@@ -714,13 +708,13 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
             double px = tx, py = ty, pz = tz, wx = vx, wy = vy, wz = vz;      // stage point and velocity
             double bx = 0, by = 0, bz = 0, cx = 0, cy = 0, cz = 0, ce = 0;    // sums over the stages
             const int ns = rk4 ? 4 : 1;
+            const bool any_emits = __any(emits);
             for (int s = 0; s < ns; ++s) {
-                if (s == 0 && __any(emits)) {
-                    total(yes, yes, cn0, true, !emits, px, py, pz, r);
+                const bool record = s == 0 && any_emits;
+                total(std::true_type{}, record, cn0, s == 0 || live, s > 0 || !emits, px, py, pz, r);
+                if (record) {
                     if (emits) emit(r);
                     if (!__any(live)) break;
-                } else {
-                    total(yes, no, cn0, s == 0 || live, true, px, py, pz, r);
                 }
                 if (!rk4) break;
                 const double wt = (s == 1 || s == 2) ? 2.0 : 1.0;
