@@ -84,6 +84,9 @@ def test_force_grid(gpu_ctx, integrator, nx, one_lane):
     d, keep = _system(0, np.random.default_rng(0))
     d.force_grid = h
     _check(gpu_ctx, [d], nx, integrator, one_lane, 8 if one_lane else 1)
+    if not one_lane:              # the waves that the kernel's registers let a SIMD hold
+        gpu_ctx.set_systems([d])
+        assert gpu_ctx.scan(_desc(nx, 0, integrator))["waves_per_simd"] == (3 if integrator == 1 else 2)
     empty, keep2 = _system(0, np.random.default_rng(0))
     gpu_ctx.set_systems([empty])
     gpu_ctx.grid_free(h)
