@@ -98,8 +98,8 @@ struct Lanes {
 //   from: a lane's a * b + (its neighbour's, rounded) is not its neighbour's sum,
 //   the lanes of a column then carry different states, and a long relaxation
 //   along a ridge drives them 1e-4 A apart.
-template <int G, int N>
-__device__ inline void group_sums(double* r, bool record) {
+template <int G, int N, bool PICK>
+__device__ inline void group_sums(double* r) {
 #pragma clang fp contract(off)
     if constexpr (G <= 8) {
 #pragma unroll
@@ -113,13 +113,13 @@ __device__ inline void group_sums(double* r, bool record) {
     } else {
         const int lane = threadIdx.x & 63;
         double d = 0.0;
-        if (record) {
+        if (PICK) {
             double row[N];
 #pragma unroll
             for (int q = 0; q < N; ++q) row[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(r[q], 1.0, 0.0, 0, 0, 0);
-            d = row[0];
-#pragma unroll
-            for (int q = 1; q < N; ++q) d = (lane & 3) == q ? row[q] : d;
+            const bool odd = lane & 1, high = lane & 2;
+            const double lo = odd ? row[1] : row[0], hi = N > 3 && odd ? row[N - 1] : row[2];
+            d = high ? hi : lo;
         } else {
 #pragma unroll
             for (int q = 0; q < N; ++q)
@@ -319,6 +319,12 @@ inline int resident_sites(int n, int G, bool mid) {
     return per <= 2 ? 2 : (per <= 6 ? per : most);
 }
 
+// A branch that one trip in a hundred takes: laid out behind the others, so that
+// the registers it needs are not spilled on their way (57 scans of all modes: 0.98 of
+// the time).  Not in the images' kernels without the midpoint step, which it costs
+// up to a third (Euler, 32 sites, 64 x 64 x 6: 1.05 -> 1.46 ms).
+#define SELDOM(branch) (IMG && !MID ? (branch) : __builtin_expect((branch), 0))
+
 // RES of a lane's sites stay in registers for the whole scan (the first RES
 // of its share, loaded from the staged copy); the others stream from LDS two
 // at a time.
@@ -473,8 +479,8 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
     };
     // tip-surface force and energy at p, summed over the group's lanes; record:
     // for some group's record
-    auto surface = [&](auto want_e, bool record, Corner& cn, bool counts, double px, double py, double pz, double* r) {
-        constexpr bool E = decltype(want_e)::value;
+    auto surface = [&](auto want_e, auto record, Corner& cn, bool counts, double px, double py, double pz, double* r) {
+        constexpr bool E = decltype(want_e)::value, PICK = decltype(record)::value;
         r[3] = 0;
         if constexpr (GRID) {
             const double w = corner(cn, counts, px, py, pz);
@@ -482,7 +488,7 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
             r[1] = w * cn.v.y;
             r[2] = w * cn.v.z;
             if (E) r[3] = w * cn.v.w;
-            group_sums<G, E ? 4 : 3>(r, record);
+            group_sums<G, E ? 4 : 3, PICK>(r);
         } else if constexpr (IMG) {
             r[0] = r[1] = r[2] = 0;
             if (has_grid && gl < 8) {   // eight of the column's lanes hold the potential's corners
@@ -513,7 +519,7 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
                 q1 = q2;
             }
             images_acc<E>(st, q1, ax, ay, pz, r);
-            group_sums<G, E ? 4 : 3>(r, record);
+            group_sums<G, E ? 4 : 3, PICK>(r);
             if (E) r[3] *= 1.0 / 12.0;
         } else {
             r[0] = r[1] = r[2] = 0;
@@ -544,7 +550,7 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
                 }
             }
             if (FLAT) r[2] *= z;
-            group_sums<G, E ? 4 : 3>(r, record);
+            group_sums<G, E ? 4 : 3, PICK>(r);
             if (E) r[3] *= COUL ? 1.0 / 3.0 : 1.0 / 12.0;
         }
     };
@@ -552,7 +558,7 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
     // contracted with the product a dummy value comes from: it would be in the call
     // whose with_d is known and not in the other, and a column's rounding would
     // depend on whether a neighbour in its wave has a record to write.
-    auto total = [&](auto want_e, bool record, Corner& cn, bool counts, bool with_d, double px, double py, double pz,
+    auto total = [&](auto want_e, auto record, Corner& cn, bool counts, bool with_d, double px, double py, double pz,
                      double* r) {
 #pragma clang fp contract(off)
         constexpr bool E = decltype(want_e)::value;
@@ -562,6 +568,8 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
 #pragma unroll
         for (int q = 0; q < (E ? 4 : 3); ++q) r[q] += with_d ? d[q] : 0.0;
     };
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
     auto begin_height = [&]() {
         n_tot = 1; dt = a.dt; alpha = 0.1; nnn = 0; flags = 0;
         mgf = mge = mgp = INFINITY;
@@ -635,7 +643,7 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
 
     for (;;) {
         // ---- groups without a column steal one from molecule m
-        if (__any(col < 0)) {
+        if (SELDOM(__any(col < 0))) {
             const bool need = leader && col == -1;
             const uint64_t need_mask = __ballot(need);
             if (need_mask) {
@@ -687,14 +695,14 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
             // half step: every running group at its tip, and the groups with a
             // finished height at theirs (tip-surface terms only)
             const double hx = dt / 2 * vx, hy = dt / 2 * vy, hz = dt / 2 * vz;
-            if (__any(emits)) {
-                total(std::true_type{}, true, cn0, true, !emits, tx, ty, tz, r);
+            if (SELDOM(__any(emits))) {
+                total(yes, yes, cn0, true, !emits, tx, ty, tz, r);
                 if (emits) emit(r);
             } else {
-                total(std::false_type{}, false, cn0, true, true, tx, ty, tz, r);
+                total(no, no, cn0, true, true, tx, ty, tz, r);
             }
             const double ax = fma(dt / 2, r[0], vx), ay = fma(dt / 2, r[1], vy), az = fma(dt / 2, r[2], vz);
-            total(std::true_type{}, false, cn1, live, true, tx + hx, ty + hy, tz + hz, r);
+            total(yes, no, cn1, live, true, tx + hx, ty + hy, tz + hz, r);
             if (live) {
                 tx = fma(dt, ax, tx); ty = fma(dt, ay, ty); tz = fma(dt, az, tz);
                 vx = fma(dt, r[0], vx); vy = fma(dt, r[1], vy); vz = fma(dt, r[2], vz);
@@ -711,8 +719,8 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
             const bool any_emits = __any(emits);
             for (int s = 0; s < ns; ++s) {
                 const bool record = s == 0 && any_emits;
-                total(std::true_type{}, record, cn0, s == 0 || live, s > 0 || !emits, px, py, pz, r);
-                if (record) {
+                total(yes, yes, cn0, s == 0 || live, s > 0 || !emits, px, py, pz, r);
+                if (SELDOM(record)) {
                     if (emits) emit(r);
                     if (!__any(live)) break;
                 }
