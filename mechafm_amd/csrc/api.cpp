@@ -700,7 +700,7 @@ static mafm_status plan_fast(mafm_ctx* c, const mafm_scan_desc* d, bool f32, con
     p.W = 1;
     if (p.iter) {
         // two waves a SIMD hold the resident sites; a force grid leaves room for three
-        // (154 registers), with SD, Euler or RK4 for two (181)
+        // (154 registers), with SD, Euler or RK4 for two (184)
         if (waves_per_simd == 0) p.wps = p.mode == 1 && mid ? 3 : 2;
         const size_t bytes = p.mode == 1 ? 1 : scan_iter_lds(p.n_min, (int)max_sites, p.G, mid, p.mode == 2);
         const long per_cu = (long)(c->lds_per_cu / bytes);

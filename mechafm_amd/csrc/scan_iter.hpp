@@ -9,22 +9,30 @@
 //   * the two evaluations of a midpoint iteration (four of RK4) follow each
 //     other in straight code, all groups of a wave in step; a group whose
 //     height is done takes its output evaluation with the others' first one;
-//   * the molecule's constants sit in scalar registers, RES sites of each lane
-//     in vector registers, the rest streams from LDS two sites ahead;
+//   * the molecule's constants are loaded once, into scalar registers as far as
+//     those go (21 to 44 values of the site kernels, 55 to 61 of the force grids',
+//     68 to 132 of the images' spill into lanes of vector registers); RES sites of
+//     each lane sit in vector registers, the rest streams from LDS two sites ahead;
 //   * groups of 16 and more lanes are summed on the FP64 matrix unit;
 //   * a force grid is read by eight lanes a column, one corner each, kept in
 //     registers until the cell changes.
 // What bounds it now: FP64 issue (4 cycles an instruction; one that needs the
 // last one's result waits 8, so two waves a SIMD fill the pipe) and, for few
-// columns, the length of the longest column's chain.
-// Measured (kernel ms, before -> now):
-//   one column over 96 sites                                      16.4 -> 3.2
-//   101 x 101 columns x 41 heights, 96 charge-free flat sites     26.5 -> 12.5 (not as flat 13.2)
-//   33 x 33 x 41, RK4, 131 charged sites                          57 -> 16
-//   128 x 128 x 36 through a force grid                           26.4 -> 7.1
-//   128 x 128 x 30, 150 charged flat sites                        54.9 -> 18.6 (20.2)
-//   64 flat molecules of 20 to 400 charged sites, 64 x 64 x 40    406 -> 361 (392)
+// columns, the length of the longest column's chain, in which an iteration's
+// evaluations follow each other although the midpoint step's two points are known
+// together (of RK4's four, the first two).  The images' kernels use all 256
+// vector registers and 84 to 112 B of scratch a lane, a few of the others 36 B.
+// Measured (kernel ms, general kernels -> now):
+//   one column over 96 sites                                      16.6 -> 3.0
+//   101 x 101 columns x 41 heights, 96 charge-free flat sites     32.2 -> 12.6
+//   33 x 33 x 41, RK4, 131 charged sites                          51 -> 16.5
+//   128 x 128 x 36 through a force grid                           24.1 -> 6.9
+//   128 x 128 x 30, 150 charged flat sites                        54.9 -> 18.3
+//   64 flat molecules of 20 to 400 charged sites, 64 x 64 x 40    402 -> 359
 //   64 x 64 x 40, 2000 sites with nine images and a potential     437 -> 244
+// (as sites of different heights the flat ones took 13.2, 20.2 and 392 where the
+// flat kernels took 12.5, 18.6 and 361).  Many columns over few sites stay with the
+// general kernels, one lane a column (one_lane_is_faster, api.cpp).
 // Tried and left out: flat or not decided in the kernel (RK4 17 -> 21: both
 // bodies' code and registers), charge-free sites sharing a reciprocal by fours
 // (the chain grows: one column 3.2 -> 3.9).
@@ -84,16 +92,18 @@ struct Lanes {
 // of them; all lanes of the wave active.
 //   G <= 8: DPP butterflies, value by value in step (three instructions a
 //   value and stage, and no wait between a write and its DPP read).
-//   G >= 16: two contractions with 0 / 1 matrices on the FP64 matrix unit.
+//   G >= 16: two contractions on the FP64 matrix unit, the first with 0 / 1 matrices.
 //   The first puts value q's sum over a block's columns into column q of one
 //   result (the values' matrices accumulate), the second adds the four rows;
 //   the sums are then in lanes 0-3 of every quad and four DPP moves hand them
 //   out.  Products with 0 and 1 are exact, except that 0 x inf is NaN: one
 //   value's infinity makes the others NaN.  An iteration is lost either way (the
-//   mixing's |f| is infinite); for the sums a record holds (record) the values'
-//   row sums are picked by lane instead, the same bits where they are finite.  16
-//   lanes, 3 values: 4 matrix instructions (16 cycles of the FP64 pipe each) and 6
-//   moves against 36 instructions of the butterflies.
+//   mixing's |f| is infinite).  PICK, for sums that a record may hold: the first
+//   product is with ones, and the lanes pick the value of their column: the same
+//   bits where they are finite; in every sum 0.999 of the time over 57 scans, but up
+//   to 4 % more for the midpoint step over few sites, whose records alone take it.
+//   16 lanes, 3 values: 4 matrix instructions (16 cycles of the FP64 pipe each) and
+//   6 moves against 36 instructions of the butterflies.
 //   No addition here may be contracted with the product a caller's value comes
 //   from: a lane's a * b + (its neighbour's, rounded) is not its neighbour's sum,
 //   the lanes of a column then carry different states, and a long relaxation
@@ -320,7 +330,7 @@ inline int resident_sites(int n, int G, bool mid) {
 }
 
 // A branch that one trip in a hundred takes: laid out behind the others, so that
-// the registers it needs are not spilled on their way (57 scans of all modes: 0.98 of
+// the registers it needs are not spilled on their way (57 scans of all modes: 0.97 of
 // the time).  Not in the images' kernels without the midpoint step, which it costs
 // up to a third (Euler, 32 sites, 64 x 64 x 6: 1.05 -> 1.46 ms).
 #define SELDOM(branch) (IMG && !MID ? (branch) : __builtin_expect((branch), 0))
@@ -617,7 +627,8 @@ __device__ __attribute__((always_inline)) inline void scan_iter_body(const ScanA
         if (track) fire_margin(p, v2, v2 > 0 ? rsq64h(v2) : 0.0, mgp);
         // |v| / |f| by one root; 0 where the force has no direction (vectors.hpp:107-114)
         // (beyond |f| = 2^200, where a tip was thrown off an atom, of the product over
-        // 2^1000: it would overflow where its factors do not)
+        // 2^1000: it would overflow where its factors do not; 0 to 2 % of an iteration,
+        // a branch to two roots 3 to 5)
         const bool thrown = f2 > 0x1p400;
         const double vf = v2 * (f2 * (thrown ? 0x1p-1000 : 1.0));
         const double s = (f2 > 1e-20 && vf > 1e-280) ? alpha * (thrown ? 0x1p-500 : 1.0) * v2 * rsq64h(vf) : 0.0;
