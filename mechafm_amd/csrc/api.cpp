@@ -553,6 +553,9 @@ static int iter_mode(const mafm_ctx* c, const std::vector<long>& cols, bool& cou
 //   molecules of 64^2 columns (each one's last columns run in waves of few): 3 to 8
 //     sites, 16 molecules 1.09, 32: 0.67, 256: 0.43; 20 to 40 sites, 32: 1.30, 64:
 //     0.98, 256: 0.86; 20 to 100 sites, 128: 1.00
+//   a large molecule among small ones, whose chain on one lane may outlast all the
+//     others' work: 63 of 6 sites and one of 200 2.24, 255 of 4 and one of 400 1.14, 200
+//     of 10 and one of 300 0.82, 120 of 6 and 8 of 100 0.60
 //   RK4: 1 site 256^2 1.03, 1000^2 0.78; 8 sites 640^2 1.04.  SD and Euler: 4 sites 128^2
 //     1.85 and 1.70, 256^2 0.86 and 0.81; 80 sites 640^2 1.04 and 1.00
 //   force grid of 76 MB: 256^2 1.08, 320^2 0.93, 1000^2 0.68 (Euler 128^2 1.47, 200^2 0.81);
@@ -562,11 +565,12 @@ static int iter_mode(const mafm_ctx* c, const std::vector<long>& cols, bool& cou
 static bool one_lane_is_faster(const mafm_ctx* c, const mafm_scan_desc* d, const std::vector<long>& cols, int mode) {
     const bool fire = d->minimiser == MAFM_MIN_FIRE, rk4 = fire && d->integrator == MAFM_INT_RK4;
     const bool staged = rk4 || (fire && d->integrator == MAFM_INT_MIDPOINT);   // more than one evaluation an iteration
-    double total = 0, sites = 0, most = 0, grid_bytes = 0;
+    double total = 0, sites = 0, largest = 0, most = 0, grid_bytes = 0;
     for (size_t m = 0; m < c->mols.size(); ++m) {
         const DevMol& M = c->mols[m];
         total += (double)cols[m];
         sites += (double)cols[m] * M.n_sites;
+        if (cols[m] > 0) largest = std::max(largest, (double)M.n_sites);
         most = std::max(most, (double)cols[m]);
         if (mode != 1 || cols[m] <= 0) continue;
         const HostGrid& g = c->grids[M.force_grid];
@@ -576,13 +580,15 @@ static bool one_lane_is_faster(const mafm_ctx* c, const mafm_scan_desc* d, const
     const double n = sites / total;
     if (mode == 1) return total >= (!staged ? 32e3 : grid_bytes > 256e6 ? 150e3 : 75e3);
     if (mode == 2) {
+        if (largest > 2 * n) return false;
         const double rho = (staged ? 1.0 : 0.7) * (170 + 62 * n) / (260 * std::ceil(n / 8) + 330);
         return total * (1 - rho) >= (staged ? 25e3 : 17e3);
     }
-    const double drain = 100 * std::min(1.0, 4096 / most);
-    double rho = (190 + 16 * n) / (45 * std::ceil(n / 4) + 330 + drain);
+    const double work = 45 * std::ceil(n / 4) + 330 + 100 * std::min(1.0, 4096 / most);
+    if (largest > 2 * n && 1400 + 56 * largest > 1.35 * total / 32768 * work) return false;
+    double rho = (190 + 16 * n) / work;
     if (rk4) rho += 0.15;
-    if (!staged) rho = 0.6 + n / (fire ? 400 : 200);
+    if (!staged) rho = 0.6 + n / (!fire ? 200 : most > 4096 ? 300 : 400);
     if (rho >= 1) return false;
     const double from = (staged && !rk4 ? 40e3 : 20e3) * (std::pow(1 - rho, -1.4) - 1.4);
     return total >= (most < 1024 ? from * std::max(1.0, n / 16) : from);

@@ -67,6 +67,14 @@ def test_sites(gpu_ctx, integrator, n, molecules, nx, one_lane):
     _check(gpu_ctx, [d for d, _ in made], nx, integrator, one_lane, 4 if one_lane else 1)
 
 
+@pytest.mark.parametrize("sizes,nx,one_lane", [([6] * 63 + [200], 64, False), ([6] * 64, 64, True),
+                                               ([6] * 60 + [100] * 4, 96, True)])
+def test_uneven_molecules(gpu_ctx, sizes, nx, one_lane):
+    rng = np.random.default_rng(len(sizes))
+    made = [_system(n, rng) for n in sizes]
+    _check(gpu_ctx, [d for d, _ in made], nx, 1, one_lane, 4 if one_lane else 1)
+
+
 @pytest.mark.parametrize("integrator,n,nx,one_lane", [(1, 2, 160, False), (1, 2, 256, True), (1, 16, 256, False),
                                                       (0, 2, 128, False), (0, 2, 176, True)])
 def test_images(gpu_ctx, integrator, n, nx, one_lane):
