@@ -558,7 +558,8 @@ static int iter_mode(const mafm_ctx* c, const std::vector<long>& cols, bool& cou
 //     of 10 and one of 300 0.82, 120 of 6 and 8 of 100 0.60
 //   RK4: 1 site 256^2 1.03, 1000^2 0.78; 8 sites 640^2 1.04.  SD and Euler: 4 sites 128^2
 //     1.85 and 1.70, 256^2 0.86 and 0.81; 80 sites 640^2 1.04 and 1.00
-//   force grid of 76 MB: 256^2 1.08, 320^2 0.93, 1000^2 0.68 (Euler 128^2 1.47, 200^2 0.81);
+//   force grid of 76 MB: 256^2 1.08, 320^2 0.94, 1000^2 0.69 (Euler 128^2 1.49, 200^2
+//     0.86; SD 200^2 1.18, 256^2 0.83);
 //     of 487 MB, past the last-level cache: 320^2 1.17, 400^2 0.99, 720^2 0.86
 //   nine images: 2 sites 192^2 1.07, 256^2 0.68; 6 sites 256^2 1.34, 640^2 0.93; 16
 //     sites 640^2 1.33
@@ -578,7 +579,7 @@ static bool one_lane_is_faster(const mafm_ctx* c, const mafm_scan_desc* d, const
     }
     if (total <= 0) return false;
     const double n = sites / total;
-    if (mode == 1) return total >= (!staged ? 32e3 : grid_bytes > 256e6 ? 150e3 : 75e3);
+    if (mode == 1) return total >= (staged ? (grid_bytes > 256e6 ? 150e3 : 75e3) : fire ? 32e3 : 50e3);
     if (mode == 2) {
         if (largest > 2 * n) return false;
         const double rho = (staged ? 1.0 : 0.7) * (170 + 62 * n) / (260 * std::ceil(n / 8) + 330);
